@@ -77,7 +77,10 @@ enum { KH_ATTN_SCALE_NONE = 0, KH_ATTN_SCALE_MUL = 1, KH_ATTN_SCALE_DIV = 2 };
 enum { KH_ROW_GENERIC = 0, KH_ROW_LAYERNORM = 1, KH_ROW_SOFTMAX = 2 };
 
 /* GEMM precisions */
-enum { KH_PREC_FP32 = 0, KH_PREC_BF16 = 1, KH_PREC_BF16X3 = 2 };
+enum { KH_PREC_FP32 = 0, KH_PREC_BF16 = 1, KH_PREC_BF16X3 = 2, KH_PREC_F16X3 = 3 };
+/* Format of a pair-stored output (kh_launch.cfg[6] of a ROW or ATTN launch; a
+ * GEMM's follows its precision). */
+enum { KH_PAIR_BF16 = 0, KH_PAIR_F16 = 1 };
 /* Prologues (kh_launch.cfg[4] of a KH_FAM_GEMV launch; LayerNorm also of a
  * KH_FAM_GEMM launch on an fp32 small-M configuration) */
 enum { KH_GEMV_PRO_NONE = 0, KH_GEMV_PRO_LAYERNORM = 1, KH_GEMV_PRO_ATTN = 2 };
@@ -205,6 +208,18 @@ typedef struct kh_pass {
  * three-pass products (cfg[5] = 2), its q, k, v together, and on the
  * three-pass GEMM configurations the A operand (bit 16) and the output of a
  * direct epilogue without split-K.
+ * fp16 pairs: an fp32 product on KH_PREC_F16X3 configurations (101-109) reads
+ * A and B as fp16 pairs: each value, scaled by a power of two into fp16's
+ * range, as h = fp16(x) and l = fp16(x - h), a row in blocks of 8 values (16
+ * bytes of h, then 16 bytes of l), 4 bytes a value, strides and offsets
+ * counted in values and multiples of 8. A . B is taken as l.h + h.l + h.h in
+ * fp32. A must be pair-stored (bit 16 of cfg[7]) with scale fparams[0]; B is
+ * the [batch][N][K'] copy (K' a multiple of 8, zero padded); refs[cfg[5]],
+ * strides 0 over M and 1 over N, is 1 / (scale of A * scale of column n),
+ * applied before the epilogue. A direct epilogue's output may be pair-stored
+ * too (also of an fp32 small-M configuration), a LayerNorm's and a blocked
+ * attention's with cfg[6] = KH_PAIR_F16: scaled by fparams[3]. Scales are
+ * powers of two; the caller guarantees that scaled values stay below 65504.
  */
 typedef struct kh_launch {
   int32_t family;

@@ -74,7 +74,8 @@ struct AttnArgs {
   int32_t mask_mode, scale_mode;
   float scale;
   int32_t o16;             // the output is bf16 (its consumer is a bf16 matmul)
-  int32_t o_pair;          // the output is pair words (its consumer is a three-pass matmul)
+  int32_t o_pair;          // the output is bf16 pair words (1) or fp16 pairs (2), as its consumer reads it
+  float o_scale;           // fp16 pairs: the power of two the output is scaled by
   uint64_t *rec;           // timeline probe only: 8 words per wave (kh_probe_attn_timeline)
 };
 
@@ -411,6 +412,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
     acc.x /= l, acc.y /= l, acc.z /= l, acc.w /= l;
     const int64_t at = b * a.o_b + (int64_t)(q0 + qr) * a.o_t + d;
+    if (a.o_pair == 2) {
+      store_f16_pairs4(a.o + b * a.o_b + (int64_t)(q0 + qr) * a.o_t, d, acc, a.o_scale);
+      continue;
+    }
     if (a.o_pair) acc = make_float4(pair_word(acc.x), pair_word(acc.y), pair_word(acc.z), pair_word(acc.w));
     if (a.o16) store_bf16x4(a.o, at, acc.x, acc.y, acc.z, acc.w);
     else *reinterpret_cast<float4 *>(a.o + at) = acc;
@@ -639,6 +644,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
     acc.x /= l, acc.y /= l, acc.z /= l, acc.w /= l;
     const int64_t at = b * a.o_b + (int64_t)(q0 + qr) * a.o_t + d;
+    if (a.o_pair == 2) {
+      store_f16_pairs4(a.o + b * a.o_b + (int64_t)(q0 + qr) * a.o_t, d, acc, a.o_scale);
+      continue;
+    }
     if (a.o_pair) acc = make_float4(pair_word(acc.x), pair_word(acc.y), pair_word(acc.z), pair_word(acc.w));
     if (a.o16) store_bf16x4(a.o, at, acc.x, acc.y, acc.z, acc.w);
     else *reinterpret_cast<float4 *>(a.o + at) = acc;
@@ -846,6 +855,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
     acc.x /= l, acc.y /= l, acc.z /= l, acc.w /= l;
     const int64_t at = b * a.o_b + (int64_t)(q0 + qr) * a.o_t + d;
+    if (a.o_pair == 2) {
+      store_f16_pairs4(a.o + b * a.o_b + (int64_t)(q0 + qr) * a.o_t, d, acc, a.o_scale);
+      continue;
+    }
     if (a.o_pair) acc = make_float4(pair_word(acc.x), pair_word(acc.y), pair_word(acc.z), pair_word(acc.w));
     if (a.o16) store_bf16x4(a.o, at, acc.x, acc.y, acc.z, acc.w);
     else *reinterpret_cast<float4 *>(a.o + at) = acc;
@@ -1161,7 +1174,12 @@ std::unique_ptr<Op> make_attn(const kh_launch &L, std::string &err, bool &unsupp
     err = "attention: pair storage only for the output of the blocked kernels";
     return nullptr;
   }
-  a.o_pair = mp >> 3 & 1;
+  a.o_pair = !(mp >> 3 & 1) ? 0 : L.cfg[6] == KH_PAIR_F16 ? 2 : 1;
+  if (a.o_pair == 2 && (a.o_b % 8 || a.o_t % 8 || L.refs[3].offset % 8 || !pow2_scale(L.fparams[3]))) {
+    err = "attention: an output of fp16 pairs needs rows of whole 32-byte blocks and a power-of-two scale";
+    return nullptr;
+  }
+  a.o_scale = L.fparams[3];
   return op;
 }
 

@@ -270,4 +270,42 @@ __device__ __forceinline__ void split_bf16x8(const float4 &x, const float4 &y, b
   lo = __builtin_bit_cast(bf16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
 }
 
+// ---------------------------------------------------------------------------
+// fp16 pairs: an fp32 value x, scaled by a power of two into fp16's range, as
+// h = fp16(x) and l = fp16(x - h), both rounded to nearest. h keeps the upper
+// 11 significant bits, the exact difference has at most 12 more and l keeps
+// 11 of them, so |x - h - l| <= 2^-23 |x| (2^-24 |x| root mean square) while
+// |x| >= 2^-1, and <= 2^-25 below (fp16 subnormals; the matrix cores keep
+// them). A product of two pairs is h.h + h.l + l.h in three fp16 MFMAs with
+// fp32 accumulation; the dropped l.l is below 2^-22 of the product.
+//
+// Storage of a row of pairs (32-byte aligned, 4 bytes a value as in fp32):
+// blocks of 8 values, 16 bytes of h then 16 bytes of l, so an MFMA operand of
+// 8 consecutive values is one 128-bit read per half.
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+  typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+  f16x2_t r;
+  r[0] = (_Float16)a, r[1] = (_Float16)b;
+  return __builtin_bit_cast(uint32_t, r);
+}
+
+// Two (scaled) values as the words of their h halves and of their l halves.
+__device__ __forceinline__ void split_f16x2(float x, float y, uint32_t &h, uint32_t &l) {
+  const _Float16 hx = (_Float16)x, hy = (_Float16)y;
+  h = pack_f16x2(x, y);
+  l = pack_f16x2(x - (float)hx, y - (float)hy);
+}
+
+// Columns [n, n + 4) (n a multiple of 4) of a row of pairs: v * scale.
+__device__ __forceinline__ void store_f16_pairs4(float *row, int64_t n, const float4 &v, float scale) {
+  uint2 h, l;
+  split_f16x2(v.x * scale, v.y * scale, h.x, l.x);
+  split_f16x2(v.z * scale, v.w * scale, h.y, l.y);
+  char *block = reinterpret_cast<char *>(row) + (n >> 3) * 32 + (n & 4) * 2;
+  *reinterpret_cast<uint2 *>(block) = h;
+  *reinterpret_cast<uint2 *>(block + 16) = l;
+}
+
 }  // namespace kh

@@ -901,7 +901,8 @@ struct TileCfg {
                                                        // 4: skinny-M direct loads ([N][K] B); 5: one
                                                        // workgroup per CU, A and B K-contiguous ([N][K] B);
                                                        // 6: small tiles, waves split K ([N][K] B); 7: bf16,
-                                                       // 64-deep steps, one tile per workgroup ([N][K] B)
+                                                       // 64-deep steps, one tile per workgroup ([N][K] B);
+                                                       // 8: fp16 pairs, one tile per workgroup ([N][K] B)
 };
 
 // Configurations by id. Ids 0-7: the copy pipeline (BK = 32, MFMA
@@ -1045,6 +1046,12 @@ constexpr TileCfg kConfigs[] = {
 #define KH_CFGBF_ROW(id, bm, bn, wm, wn, ns) {bm, bn, 64, wm, wn, 1, 16, 7, ns, KH_PREC_BF16},
     KH_GEMM_BF_CONFIGS(KH_CFGBF_ROW)
 #undef KH_CFGBF_ROW
+#define KH_CFGF16_ROW(id, bm, bn, wm, wn, ns) {bm, bn, 32, wm, wn, 1, 16, 8, ns, KH_PREC_F16X3},
+    KH_GEMM_F16_CONFIGS(KH_CFGF16_ROW)
+#undef KH_CFGF16_ROW
+#define KH_CFGSMF_ROW(id, bm, bn, wk, ns, prec) {bm, bn, 32, 1, 1, wk, 16, 6, ns, KH_PREC_F16X3},
+    KH_GEMM_SMALL_F16_CONFIGS(KH_CFGSMF_ROW)
+#undef KH_CFGSMF_ROW
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -1057,7 +1064,7 @@ constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 // GPU): 2048x3072x768 on the 32x64 tile 5% faster, the others within 1%.
 int tile_group(const TileCfg &t, int tiles_m) {
   const int lds = t.kind == 6   ? 4 * t.stages * t.bk * (t.bm + t.bn) * t.wk   // (fp32 bound)
-                  : t.kind == 5 ? 4 * t.stages * t.bk * (t.bm + t.bn)   // (fp32 bound)
+                  : t.kind == 5 || t.kind == 8 ? 4 * t.stages * t.bk * (t.bm + t.bn)   // (fp32 bound)
                   : t.kind == 7 ? t.stages * t.bk * (4 * t.bm + 2 * t.bn)
                   : t.kind == 3 ? 4 * t.stages * (t.bm * t.bk + (t.prec == KH_PREC_FP32 ? t.bk * t.bn
                                                                  : t.bn * t.bk / 2 * (t.prec == KH_PREC_BF16X3 ? 2 : 1)))
@@ -1074,6 +1081,7 @@ int tile_group(const TileCfg &t, int tiles_m) {
 hipError_t launch_config(int id, const GemmArgs &a, dim3 grid, hipStream_t stream) {
   if (kConfigs[id].kind == 5) return launch_gemm_nt(id, a, grid, stream);
   if (kConfigs[id].kind == 7) return launch_gemm_bf(id, a, grid, stream);
+  if (kConfigs[id].kind == 8) return launch_gemm_f16(id, a, grid, stream);
   if (kConfigs[id].kind == 6) return launch_gemm_small(id, a, grid, stream);
   switch (id) {
 #define KH_CFGS_CASE(cid, bm, bn, wk, depth)                                                            \
@@ -1307,7 +1315,8 @@ std::unique_ptr<Op> make_gemm(const kh_launch &L, std::string &err, bool &unsupp
     err = "matmul: unknown tile configuration " + std::to_string(cfg);
     return nullptr;
   }
-  if (L.cfg[3] != KH_PREC_FP32 && L.cfg[3] != KH_PREC_BF16 && L.cfg[3] != KH_PREC_BF16X3) {
+  if (L.cfg[3] != KH_PREC_FP32 && L.cfg[3] != KH_PREC_BF16 && L.cfg[3] != KH_PREC_BF16X3 &&
+      L.cfg[3] != KH_PREC_F16X3) {
     unsupported = true;
     err = "matmul: precision not compiled into this library";
     return nullptr;
@@ -1376,13 +1385,28 @@ std::unique_ptr<Op> make_gemm(const kh_launch &L, std::string &err, bool &unsupp
     }
     op->b_vec_layout = true;
   }
-  if (t.kind == 4 || t.kind == 5 || t.kind == 6 || t.kind == 7) {
+  a.d_cs = -1, a.o_scale = 1.0f;
+  if (t.prec == KH_PREC_F16X3) {
+    // A in pair storage (checked below with the rest of cfg[7]), rows of
+    // whole 32-byte blocks; refs[cfg[5]] the columns' powers of two
+    const int r = L.cfg[5];
+    if (r < 2 || r >= L.n_refs || L.refs[r].strides[1] != 0 || L.refs[r].strides[2] != 1) {
+      err = "matmul: fp16 pairs need the column scales as an operand with strides 0 over M, 1 over N";
+      return nullptr;
+    }
+    if (a.sa_m % 8 || a.sa_b % 8 || L.refs[0].offset % 8 || a.sb_n % 8 || a.sb_b % 8 || L.refs[1].offset % 8) {
+      err = "matmul: fp16 pair operands need rows of whole 32-byte blocks";
+      return nullptr;
+    }
+    a.d_cs = r - 2;
+  }
+  if (t.kind == 4 || t.kind == 5 || t.kind == 6 || t.kind == 7 || t.kind == 8) {
     // skinny-M direct loads / K-contiguous pipelines: A row-major with unit K
     // stride, B the [batch][N][K] copy, both read as whole 16-byte pieces; K
     // is not split across workgroups (and is a positive whole number of
-    // steps, 32 or 64 deep, for kinds 5 and 6)
+    // steps, 32 or 64 deep, for kinds 5 to 8)
     const kh_ref &ra = L.refs[0], &rb = L.refs[1];
-    const bool steps = t.kind == 5 || t.kind == 6 || t.kind == 7;
+    const bool steps = t.kind >= 5;
     const int step = steps ? t.bk : 4;
     op->b_vec_layout = a.sb_k == 1 && rb.offset % 4 == 0 && a.sb_n % 4 == 0 && a.sb_b % 4 == 0 && a.sb_n >= K;
     if (!op->a_vec_layout || !op->b_vec_layout || K % step || (steps && K == 0) || ra.offset % 4) {
@@ -1463,15 +1487,29 @@ std::unique_ptr<Op> make_gemm(const kh_launch &L, std::string &err, bool &unsupp
   if (mp) {
     const bool ap = mp & 1u, op_ = a.direct && (mp >> (2 + a.d_out) & 1u);
     const uint32_t known = (ap ? 1u : 0u) | (op_ ? 1u << (2 + a.d_out) : 0u);
-    const bool kind_ok = tr.kind == 3 || tr.kind == 5 || tr.kind == 6;
-    if (mp != known || m16 || cfg_run != cfg || t.prec != KH_PREC_BF16X3 || !kind_ok || a.pro != KH_GEMV_PRO_NONE ||
-        (op_ && a.splitk != 1)) {
+    // (fp16 pairs: of an fp32 small-M product only the output)
+    const bool f16 = t.prec == KH_PREC_F16X3 || (t.prec == KH_PREC_FP32 && tr.kind == 6 && !ap);
+    const bool kind_ok = tr.kind == 3 || tr.kind == 5 || tr.kind == 6 || tr.kind == 8;
+    if (mp != known || m16 || cfg_run != cfg || (t.prec != KH_PREC_BF16X3 && !f16) || !kind_ok ||
+        (a.pro != KH_GEMV_PRO_NONE && !f16) || (op_ && a.splitk != 1)) {
       unsupported = true;
       err = "matmul: pair storage only for A and a direct epilogue's output of a three-pass configuration "
             "(the output without split-K)";
       return nullptr;
     }
-    a.a_pair = ap ? 1 : 0, a.o_pair = op_ ? 1 : 0;
+    if (f16 && op_) {
+      const int64_t *st = a.estride[a.d_out];
+      if (st[2] != 1 || st[1] % 8 || st[0] % 8 || L.refs[2 + a.d_out].offset % 8 || N % 8 || !pow2_scale(L.fparams[3])) {
+        err = "matmul: an output of fp16 pairs needs rows of whole 32-byte blocks and a power-of-two scale";
+        return nullptr;
+      }
+      a.o_scale = L.fparams[3];
+    }
+    a.a_pair = ap ? 1 : 0, a.o_pair = !op_ ? kPairNone : f16 ? kPairF16 : kPairBf16;
+  }
+  if (t.prec == KH_PREC_F16X3 && (!a.a_pair || !pow2_scale(L.fparams[0]))) {
+    err = "matmul: fp16 pairs need A in pair storage and its power-of-two scale";
+    return nullptr;
   }
   const int64_t n_tiles = (int64_t)a.tiles_m * a.tiles_n;
   if (n_tiles >= (1ll << 31)) {

@@ -41,8 +41,14 @@ struct GemmArgs {
   int32_t a16, o16;
   // pair storage (three-pass configurations): A holds pair words; the direct
   // epilogue writes its output as pair words
-  int32_t a_pair, o_pair;
+  int32_t a_pair, o_pair;   // o_pair: kPairBf16 or kPairF16
+  // fp16 pairs (KH_PREC_F16X3): epilogue operand of the per-column power of
+  // two that takes the scaled operands' products back, and the power of two
+  // that a pair-stored output is scaled by
+  int32_t d_cs;
+  float o_scale;
 };
+enum { kPairNone = 0, kPairBf16 = 1, kPairF16 = 2 };
 
 // Run the epilogue tape for columns [n, n + valid) of output row (b, m);
 // slot 0 starts as the accumulator values. Epilogue tapes use at most 8 slots.
@@ -172,6 +178,18 @@ inline hipError_t launch_splitk_reduce(const GemmArgs &a, int cus, hipStream_t s
   X(99, 64, 64, 2, 2, 3)               \
   X(100, 128, 96, 2, 2, 3)
 
+// Configurations of the fp16-pair kernel (kind 8, kh_gemm_f16.hip; one tile
+// per workgroup): id, BM x BN, waves WM x WN, stages NS.
+#define KH_GEMM_F16_CONFIGS(X) \
+  X(101, 128, 192, 2, 4, 3)    \
+  X(102, 64, 96, 2, 2, 3)      \
+  X(103, 64, 64, 2, 2, 2)      \
+  X(104, 32, 96, 2, 2, 4)      \
+  X(105, 32, 64, 2, 2, 4)
+
+// Launch configuration `id` of kind 8 (hipErrorInvalidValue for another id).
+hipError_t launch_gemm_f16(int id, const GemmArgs &a, dim3 grid, hipStream_t stream);
+
 // Launch configuration `id` of kind 5 (hipErrorInvalidValue for another id).
 hipError_t launch_gemm_nt(int id, const GemmArgs &a, dim3 grid, hipStream_t stream);
 // Launch configuration `id` of kind 7 (hipErrorInvalidValue for another id).
@@ -182,7 +200,7 @@ constexpr int kLnMaxK = 1024;
 
 // Configurations of the small-M kernel (kind 6, kh_gemm_small.hip): id, tile
 // BM x BN, WK waves splitting K (each with a private LDS ring), NS stages,
-// precision (0 fp32, 1 bf16, 2 three-pass bf16).
+// precision (0 fp32, 1 bf16, 2 three-pass bf16, 3 fp16 pairs).
 #define KH_GEMM_SMALL_CONFIGS(X) \
   X(65, 16, 32, 4, 3, 0)         \
   X(66, 16, 32, 4, 2, 0)         \
@@ -206,6 +224,13 @@ constexpr int kLnMaxK = 1024;
   X(84, 16, 16, 8, 2, 1)         \
   X(85, 32, 32, 8, 2, 1)         \
   X(86, 16, 16, 8, 2, 2)
+
+// The same kernel over fp16 pairs (precision 3).
+#define KH_GEMM_SMALL_F16_CONFIGS(X) \
+  X(106, 16, 32, 8, 2, 3)            \
+  X(107, 32, 32, 4, 2, 3)            \
+  X(108, 32, 48, 4, 2, 3)            \
+  X(109, 16, 16, 4, 2, 3)
 
 // Launch configuration `id` of kind 6 (hipErrorInvalidValue for another id).
 hipError_t launch_gemm_small(int id, const GemmArgs &a, dim3 grid, hipStream_t stream);

@@ -1,7 +1,7 @@
 // kh_gemm_small.hip - matmul for products with few rows (configuration kind
 // 6): C[b] = epilogue(A[b] @ B[b]) with A [.., M, K] row-major fp32 and B the
 // [batch][N][K] copy of a constant weight (fp32, or the bf16 / three-pass
-// bf16 copies), both K-contiguous.
+// bf16 / fp16-pair copies), both K-contiguous.
 //
 // Same contract as the rest of the matmul family (the reference's tl.dot
 // kernel with fused epilogue, kiln/gpu/codegen.py:484-530). A product with a
@@ -62,13 +62,17 @@ namespace {
 // fragments are read, one v_mfma_f32_16x16x32_bf16 per block and step, fp32
 // accumulation (the arithmetic of the other bf16 GEMMs); 2 three-pass bf16 -
 // B the [batch][N][2K'] copy holding bf16(w) then bf16(w - bf16(w)) per row,
-// A split the same way, a.b = a_lo.b_hi + a_hi.b_lo + a_hi.b_hi.
+// A split the same way, a.b = a_lo.b_hi + a_hi.b_lo + a_hi.b_hi; 3 fp16
+// pairs (kh_common.hpp) - A and the [batch][N][K'] copy of B both hold blocks
+// of 8 values as 16 bytes of h and 16 of l, laid out and copied like fp32
+// rows, a.b = l.h + h.l + h.h on v_mfma_f32_16x16x32_f16 (48 matrix cycles
+// per block and step against 256), times the column's power of two.
 template <int BM, int BN, int WK, int NS, int PREC, bool LN>
 __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
   constexpr int BK = 32, MT = 16, ACH = BK / 4;
   constexpr int FM = BM / MT, FN = BN / MT;
-  constexpr bool BF = PREC != 0;
-  static_assert(!LN || (!BF && BM % WK == 0 && BM / WK <= 4), "LayerNorm prologue: fp32, at most 4 rows per wave");
+  constexpr bool BF = PREC == 1 || PREC == 2;
+  static_assert(!LN || (PREC == 0 && BM % WK == 0 && BM / WK <= 4), "LayerNorm prologue: fp32, at most 4 rows per wave");
   constexpr int B_HALF = BN * BK / 2;           // words of one bf16 copy of a stage's B rows
   constexpr int A_FLOATS = BM * BK;
   constexpr int STAGE = A_FLOATS + (BF ? B_HALF * (PREC == 2 ? 2 : 1) : BN * BK);   // words: A rows, then B rows
@@ -167,11 +171,11 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
     }
   }
 
-  f32x4 acc[FM][FN];
+  f32x4 acc[FM][FN], acc_small[FM][FN];   // (acc_small: PREC 3)
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
-    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = acc_small[fm][fn] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto part = [](const float4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
 
   for (int p = 0; p < NS - 1 && p < n_steps; ++p) issue(p);
@@ -265,6 +269,19 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
           }
           acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[fm], bh, acc[fm][fn], 0, 0, 0);
         }
+    } else if constexpr (PREC == 3) {
+      // chunk 2g is h, chunk 2g + 1 is l; the small products accumulate apart
+      // (their roundings are then 2^-11 of the sum's)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+          for (int fn = 0; fn < FN; ++fn) {
+            f32x4 &c = p < 2 ? acc_small[fm][fn] : acc[fm][fn];
+            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8_t *>(&xa[fm][p == 0]),
+                                                       *reinterpret_cast<const f16x8_t *>(&xb[fn][p == 1]), c, 0, 0, 0);
+          }
     } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -296,8 +313,8 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
     for (int i = 0; i < valid; ++i) v[i] = p[(int64_t)(n + i) * a.estride[j][2]];
     return make_float4(v[0], v[1], v[2], v[3]);
   };
-  float4 pre_b = make_float4(0.f, 0.f, 0.f, 0.f), pre_r = pre_b, pre_g = pre_b, pre_c = pre_b;
-  if ((a.direct || LN) && q0 < GROUPS) {
+  float4 pre_b = make_float4(0.f, 0.f, 0.f, 0.f), pre_r = pre_b, pre_g = pre_b, pre_c = pre_b, pre_s = pre_b;
+  if ((a.direct || LN || PREC == 3) && q0 < GROUPS) {
     int m, n;
     group_mn(q0, m, n);
     if (m < a.M && n < a.N) {
@@ -306,6 +323,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
         pre_g = load4(a.pro_g, m, n, valid);
         if (a.pro_b >= 0) pre_c = load4(a.pro_b, m, n, valid);
       }
+      if constexpr (PREC == 3) pre_s = load4(a.d_cs, m, n, valid);   // the columns' powers of two
       if (a.direct && a.d_bias >= 0) pre_b = load4(a.d_bias, m, n, valid);
       if (a.direct && a.d_res >= 0) pre_r = load4(a.d_res, m, n, valid);
     }
@@ -319,7 +337,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mine[(fm * MT + 4 * g + i) * CS + fn * MT + li] = acc[fm][fn][i];
+      for (int i = 0; i < 4; ++i) mine[(fm * MT + 4 * g + i) * CS + fn * MT + li] = acc[fm][fn][i] + (PREC == 3 ? acc_small[fm][fn][i] : 0.0f);
   if constexpr (LN) {
     // the row's statistics over this wave's K range: lanes li, li + 16,
     // li + 32, li + 48 merged (lane group 0's result kept)
@@ -367,6 +385,10 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
         sum.x += c.x, sum.y += c.y, sum.z += c.z, sum.w += c.w;
       }
     }
+    if constexpr (PREC == 3) {
+      const float4 cs = q == q0 ? pre_s : load4(a.d_cs, m, n, valid);
+      sum.x *= cs.x, sum.y *= cs.y, sum.z *= cs.z, sum.w *= cs.w;
+    }
     if (!a.direct) {
       Vec<4> v;
       v.v[0] = sum.x, v.v[1] = sum.y, v.v[2] = sum.z, v.v[3] = sum.w;
@@ -385,12 +407,14 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
       else if (a.d_act == KH_OP_GELU_ERF) v[i] = op_gelu_erf(v[i]);
       else if (a.d_act == KH_OP_RELU) v[i] = v[i] != v[i] ? v[i] : fmaxf(v[i], 0.0f);
     }
-    if (a.o_pair) {
+    if (PREC == 2 && a.o_pair) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = pair_word(v[i]);
     }
     float *o = a.eptr[a.d_out] + (int64_t)bidx * a.estride[a.d_out][0] + (int64_t)m * a.estride[a.d_out][1];
-    if ((a.e_vec_mask >> a.d_out & 1) && valid == 4) {
+    if ((PREC == 0 || PREC == 3) && a.o_pair) {   // (fp16 pairs)
+      store_f16_pairs4(o, n, make_float4(v[0], v[1], v[2], v[3]), a.o_scale);
+    } else if ((a.e_vec_mask >> a.d_out & 1) && valid == 4) {
       *reinterpret_cast<float4 *>(o + n) = make_float4(v[0], v[1], v[2], v[3]);
     } else {
       for (int i = 0; i < valid; ++i) o[(int64_t)(n + i) * a.estride[a.d_out][2]] = v[i];
@@ -414,6 +438,7 @@ hipError_t launch_gemm_small(int id, const GemmArgs &a, dim3 grid, hipStream_t s
     }                                                                                                       \
     break;
     KH_GEMM_SMALL_CONFIGS(KH_CFGSM_CASE)
+    KH_GEMM_SMALL_F16_CONFIGS(KH_CFGSM_CASE)
 #undef KH_CFGSM_CASE
     default: return hipErrorInvalidValue;
   }

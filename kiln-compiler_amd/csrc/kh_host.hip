@@ -335,6 +335,9 @@ void host_matmul(const kh_launch &L, float *const *p) {
   for (int64_t b = 0; b < batch; ++b)
     for (int64_t m = 0; m < M; ++m) {
       a_row(L, p, b, m, row);
+      // fp16 pairs: an activation's pair storage is its fp32 value here, split as its producer would
+      if (prec == KH_PREC_F16X3)
+        for (float &x : row) x *= L.fparams[0];
       for (int64_t n = 0; n < N; ++n) {
         double acc = 0.0;
         for (int64_t k = 0; k < K; ++k) {
@@ -344,6 +347,11 @@ void host_matmul(const kh_launch &L, float *const *p) {
             acc += (double)a * (double)p[1][at];
           } else if (prec == KH_PREC_BF16) {
             acc += (double)bf16_round(a) * (double)bf16_value(b16[at]);
+          } else if (prec == KH_PREC_F16X3) {   // fp16 pairs: l.h + h.l + h.h, B in blocks of 8 h and 8 l
+            const _Float16 *w = reinterpret_cast<const _Float16 *>(p[1]) + 2 * (at - k % 8) + k % 8;
+            const double wh = (double)w[0], wl = (double)w[8];
+            const _Float16 ah = (_Float16)a, al = (_Float16)(a - (float)ah);
+            acc += (double)al * wh + (double)ah * wl + (double)ah * wh;
           } else {   // three products of bf16 halves: lo*hi + hi*lo + hi*hi
             const float a_hi = bf16_round(a);
             const float a_lo = std::isfinite(a_hi) ? bf16_round(a - a_hi) : 0.0f;
@@ -355,6 +363,7 @@ void host_matmul(const kh_launch &L, float *const *p) {
         // a GEMM's LayerNorm prologue: the folded beta . W, per column
         const int c_ref = L.family == KH_FAM_GEMM && L.cfg[4] == KH_GEMV_PRO_LAYERNORM ? L.cfg[6] : -1;
         if (c_ref >= 0) acc += (double)p[c_ref][offset_of(L.refs[c_ref], idx, 3)];
+        if (prec == KH_PREC_F16X3) acc *= (double)p[L.cfg[5]][offset_of(L.refs[L.cfg[5]], idx, 3)];
         slot[0] = (float)acc;
         const Operands mem(L, p);
         run_tape(

@@ -4,6 +4,7 @@
 // patches the resolved device pointers and launches.
 #pragma once
 
+#include <cmath>
 #include <hip/hip_runtime.h>
 
 #include <memory>
@@ -82,6 +83,13 @@ inline uint32_t bf16_refs(const kh_launch &L) {
 inline uint32_t pair_refs(const kh_launch &L) {
   const bool fam = L.family == KH_FAM_ROW || L.family == KH_FAM_ATTN || L.family == KH_FAM_GEMM;
   return fam ? ((uint32_t)L.cfg[7] >> 16) & ((1u << KH_MAX_REFS) - 1) : 0u;
+}
+
+// fp16 pair storage: the power of two a value is scaled by before it is split
+// (kh_common.hpp).
+inline bool pow2_scale(float s) {
+  int e;
+  return std::isfinite(s) && s > 0.0f && std::frexp(s, &e) == 0.5f;
 }
 
 // Each factory returns nullptr and sets `err` when the descriptor is invalid or

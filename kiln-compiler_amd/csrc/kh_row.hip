@@ -38,7 +38,8 @@ struct LnArgs {
   uint32_t rows, inner;
   float inv_n1, inv_n2, eps;
   int32_t out16;        // the output is bf16 (its consumer is a bf16 matmul)
-  int32_t out_pair;     // the output is pair words (its consumer is a three-pass matmul)
+  int32_t out_pair;     // the output is bf16 pair words (1) or fp16 pairs (2), as its consumer reads it
+  float out_scale;      // fp16 pairs: the power of two the output is scaled by
 };
 
 // One row per wave and no grid-stride loop: the grid covers every row, so
@@ -85,6 +86,10 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const LnArgs a) {
         if (a.beta) {
           const float4 b = *reinterpret_cast<const float4 *>(a.beta + c);
           y.x += b.x, y.y += b.y, y.z += b.z, y.w += b.w;
+        }
+        if (a.out_pair == 2) {
+          store_f16_pairs4(a.out + (int64_t)row * a.out_rs, c, y, a.out_scale);
+          continue;
         }
         if (a.out_pair) y = make_float4(pair_word(y.x), pair_word(y.y), pair_word(y.z), pair_word(y.w));
         if (a.out16) store_bf16x4(a.out, (int64_t)row * a.out_rs + c, y.x, y.y, y.z, y.w);
@@ -452,7 +457,13 @@ std::unique_ptr<Op> make_row(const kh_launch &L, std::string &err, bool &unsuppo
           err = "row: pair storage only for a LayerNorm's output";
           return nullptr;
         }
-        op->args.out_pair = mp ? 1 : 0;
+        op->args.out_pair = !mp ? 0 : L.cfg[6] == KH_PAIR_F16 ? 2 : 1;
+        if (op->args.out_pair == 2 &&
+            (inner % 8 || rs[out] % 8 || L.refs[out].offset % 8 || !pow2_scale(L.fparams[3]))) {
+          err = "row: an output of fp16 pairs needs rows of whole 32-byte blocks and a power-of-two scale";
+          return nullptr;
+        }
+        op->args.out_scale = L.fparams[3];
         return op;
       }
     }

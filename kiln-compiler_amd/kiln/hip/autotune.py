@@ -162,6 +162,17 @@ TILES = {
     98: (64, 96, 64, 2, 2, 1, 16),
     99: (64, 64, 64, 2, 2, 1, 16),
     100: (128, 96, 64, 2, 2, 1, 16),
+    # fp32 products on fp16 pairs: one tile per workgroup (101-105), and the
+    # small-M kernel (106-109)
+    101: (128, 192, 32, 2, 4, 1, 16),
+    102: (64, 96, 32, 2, 2, 1, 16),
+    103: (64, 64, 32, 2, 2, 1, 16),
+    104: (32, 96, 32, 2, 2, 1, 16),
+    105: (32, 64, 32, 2, 2, 1, 16),
+    106: (16, 32, 32, 1, 1, 8, 16),
+    107: (32, 32, 32, 1, 1, 4, 16),
+    108: (32, 48, 32, 1, 1, 4, 16),
+    109: (16, 16, 32, 1, 1, 4, 16),
 }
 # configurations of the skinny-M kernel: A row-major with unit K stride and
 # K % 4 == 0, B a constant read through its [batch][N][K] copy, no split-K;
@@ -170,7 +181,7 @@ TILES = {
 SKINNY = frozenset(range(47, 55))
 # configurations of the K-contiguous pipeline: A as for the skinny kernel, B
 # the [batch][N][K] copy of a constant, K a multiple of 32, no split-K
-K_CONTIGUOUS = frozenset(range(55, 65)) | frozenset(range(87, 101))
+K_CONTIGUOUS = frozenset(range(55, 65)) | frozenset(range(87, 106))
 # the bf16 configurations with 64-deep K steps (kind 7): they also read A as
 # bf16 when its producer stores it that way (kiln/hip/lowering.py,
 # plan_bf16_storage)
@@ -178,7 +189,7 @@ BF16_A = frozenset(range(95, 101))
 # configurations of the small-M kernel: as the K-contiguous pipeline (B the
 # [batch][N][K] copy, K a positive multiple of 32, no split-K), for products
 # with at most SMALL_M_MAX rows
-SMALL_M = frozenset(range(65, 87))
+SMALL_M = frozenset(range(65, 87)) | frozenset(range(106, 110))
 SMALL_M_MAX = 1024
 # configurations that read B through its [batch][N][K] copy
 NK_B = SKINNY | K_CONTIGUOUS | SMALL_M
@@ -192,6 +203,7 @@ SKINNY_TURNS = 4
 PRECISION = {t: ("bf16" if 15 <= t <= 20 or 34 <= t <= 41 or 75 <= t <= 79 or t in (84, 85) or 87 <= t <= 91
                  or 95 <= t <= 100
                  else "bf16x3" if 26 <= t <= 31 or 42 <= t <= 45 or 80 <= t <= 83 or t == 86 or 92 <= t <= 94
+                 else "f16x3" if t >= 101
                  else "fp32")
              for t in TILES}
 # workgroups of each configuration one CU holds at once (LDS / VGPR bound,
@@ -206,7 +218,8 @@ OCCUPANCY = {0: 2, 1: 2, 2: 3, 3: 2, 4: 4, 5: 2, 6: 1, 7: 1, 8: 4, 9: 4, 10: 4, 
              65: 2, 66: 3, 67: 3, 68: 1, 69: 2, 70: 1, 71: 2, 72: 1, 73: 1, 74: 4,
              75: 4, 76: 2, 77: 3, 78: 3, 79: 4, 80: 3, 81: 2, 82: 2, 83: 4, 84: 2, 85: 1, 86: 2,
              87: 1, 88: 1, 89: 1, 90: 1, 91: 1, 92: 1, 93: 1, 94: 1,
-             95: 1, 96: 1, 97: 1, 98: 1, 99: 1, 100: 1}
+             95: 1, 96: 1, 97: 1, 98: 1, 99: 1, 100: 1,
+             101: 1, 102: 2, 103: 3, 104: 2, 105: 3, 106: 1, 107: 2, 108: 2, 109: 4}
 EFFICIENCY = {0: 0.62, 1: 0.6, 2: 0.62, 3: 0.58, 4: 0.66, 5: 0.62, 6: 0.67, 7: 0.55,
               8: 0.55, 9: 0.55, 10: 0.5, 11: 0.5, 12: 0.45, 13: 0.5, 14: 0.55,
               15: 0.15, 16: 0.15, 17: 0.15, 18: 0.15, 19: 0.15, 20: 0.15,
@@ -220,9 +233,20 @@ EFFICIENCY = {0: 0.62, 1: 0.6, 2: 0.62, 3: 0.58, 4: 0.66, 5: 0.62, 6: 0.67, 7: 0
               75: 0.12, 76: 0.12, 77: 0.12, 78: 0.12, 79: 0.1, 80: 0.25, 81: 0.25, 82: 0.25, 83: 0.2,
               84: 0.1, 85: 0.12, 86: 0.2,
               87: 0.2, 88: 0.2, 89: 0.2, 90: 0.2, 91: 0.2, 92: 0.35, 93: 0.35, 94: 0.35,
-              95: 0.3, 96: 0.28, 97: 0.26, 98: 0.26, 99: 0.25, 100: 0.26}
+              95: 0.3, 96: 0.28, 97: 0.26, 98: 0.26, 99: 0.25, 100: 0.26,
+              **{t: 0.35 for t in range(101, 110)}}
+# Measured times of the fp16-pair configurations (GPT-2 shapes, M 128 to 2048,
+# K 768 and 3072): microseconds a launch takes beyond its K steps (launch,
+# first loads, output), and microseconds per 32-deep step for every tile that
+# falls to a CU (the matrix cores, the copies into LDS and the tiles sharing
+# the CU go at that rate whatever their number)
+F16_TIMES = {101: (9.5, 0.97), 102: (6.0, 0.31), 103: (5.5, 0.20), 104: (5.5, 0.17), 105: (4.5, 0.13),
+             106: (3.4, 0.047), 107: (3.2, 0.086), 108: (4.6, 0.125), 109: (3.3, 0.031)}
+# the one whose products sum in a single chain (the others keep the small
+# products apart): for as many rows as the fp32 kernels summed so themselves
+F16_SINGLE_CHAIN = 101
 # MFMA rate of a CU relative to fp32, per precision
-RATE = {"fp32": 1.0, "bf16": 16.0, "bf16x3": 16.0 / 3}
+RATE = {"fp32": 1.0, "bf16": 16.0, "bf16x3": 16.0 / 3, "f16x3": 16.0 / 3}
 CU_MFLOP_PER_US = 0.614          # fp32 MFMA: 256 flop/clk/CU at 2.4 GHz
 ROUND_OVERHEAD_US = 8.0          # launch, prologue and epilogue of one round of workgroups
 REDUCE_US = 3.0                  # split-K reduce kernel launch
@@ -261,7 +285,7 @@ def k_major_fits(m, k, tile) -> bool:
     product with m rows and depth k."""
     if tile in SKINNY:
         return skinny_fits(m, k, tile)
-    if tile in SMALL_M and m > SMALL_M_MAX:
+    if tile in SMALL_M and m > SMALL_M_MAX or tile == F16_SINGLE_CHAIN and m <= SMALL_M_MAX:
         return False
     return k % TILES[tile][2] == 0 and k > 0
 
@@ -277,6 +301,11 @@ def estimate(tile, splitk, batch, m, n, k, cus) -> float:  # noqa: C901
     overhead, plus the MFMA time of the busiest CU (its workgroups share the
     CU's matrix cores), plus the split-K reduce (partials through HBM)."""
     bm, bn, bk = TILES[tile][:3]
+    if tile in F16_TIMES:
+        launch, step = F16_TIMES[tile]
+        tiles = math.ceil(m / bm) * math.ceil(n / bn) * batch
+        rounds = math.ceil(tiles / (cus * OCCUPANCY[tile]))
+        return launch * rounds + math.ceil(tiles / cus) * math.ceil(k / bk) * step
     units = math.ceil(m / bm) * math.ceil(n / bn) * batch * splitk
     rounds = math.ceil(units / (cus * OCCUPANCY[tile]))
     kper = math.ceil(k / splitk / bk) * bk
@@ -288,15 +317,21 @@ def estimate(tile, splitk, batch, m, n, k, cus) -> float:  # noqa: C901
     return t
 
 
-def default_matmul_config(graph, kernel, cus=None) -> dict:
-    """Tile and split-K for a matmul kernel, without measuring.
+def default_matmul_config(graph, kernel, cus=None, f16=False) -> dict:
+    """Tile and split-K for a matmul kernel, without measuring (f16: on fp16
+    pairs).
 
     Prefer the largest tile that gives every CU a workgroup; when no tile can
     (M = 128 shapes on 256 CUs), pick the tile / split-K pair with the lowest
     modelled time.
     """
     batch, m, n, k = matmul_shape(kernel)
-    return default_config_for(batch, m, n, k, cus)
+    return default_config_for(batch, m, n, k, cus, precision="f16x3" if f16 else "fp32")
+
+
+# a caller's fn(graph, kernel) takes two arguments; the lowering asks these two
+# for fp32 products on fp16 pairs too
+default_matmul_config.accepts_f16 = True
 
 
 def default_config_for(batch, m, n, k, cus=None, precision="fp32", skinny=True) -> dict:
@@ -320,7 +355,7 @@ def default_config_for(batch, m, n, k, cus=None, precision="fp32", skinny=True) 
             if best is None or t < best[0]:
                 best = (t, tile, s)
     if best is None:
-        return {"tile": {"fp32": 11, "bf16": 19, "bf16x3": 30}[precision], "splitk": 1}
+        return {"tile": {"fp32": 11, "bf16": 19, "bf16x3": 30, "f16x3": 105}[precision], "splitk": 1}
     return {"tile": best[1], "splitk": best[2]}
 
 
@@ -457,44 +492,48 @@ class GPUAutotuner:
         except OSError as err:
             warnings.warn(f"Kiln: couldn't write the GPU autotune cache ({err})")
 
-    def config_for(self, graph, kernel, a16=False):
+    def config_for(self, graph, kernel, a16=False, f16=False):
         """The configuration for ``kernel``'s matmul: cached, shipped, or
         measured now (and cached). Every answer is logged. a16: the plan can
         store the product's A operand as bf16 (bf16: its producer rounds it)
         or as pair words (bf16x3: its producer splits it), so candidates are
-        timed that way and keyed apart."""
+        timed that way and keyed apart. f16: an fp32 product that the plan
+        runs on fp16 pairs (precision "f16x3")."""
         batch, m, n, k = matmul_shape(kernel)
+        precision = "f16x3" if f16 else self.precision
         a16 = bool(a16) and self.precision in ("bf16", "bf16x3")
-        key = f"{self.device_key()}|{self.precision}{'+a16' if a16 else ''}|{batch}x{m}x{n}x{k}"
+        key = f"{self.device_key()}|{precision}{'+a16' if a16 else ''}|{batch}x{m}x{n}x{k}"
         if a16 and self.precision == "bf16x3" and not any(_usable(t.get(key)) for t in (self._cache, self._shipped)):
             # three-pass products reading pair-stored A: timed that way only
             # ahead of time (tune_shipped), else the plain entry
             a16 = False
-            key = f"{self.device_key()}|{self.precision}|{batch}x{m}x{n}x{k}"
+            key = f"{self.device_key()}|{precision}|{batch}x{m}x{n}x{k}"
         for source, table in (("cache", self._cache), ("shipped", self._shipped)):
             if _usable(table.get(key)):
                 entry = table[key]
                 break
         else:
             source = "tuned"
-            entry = self.tune(batch, m, n, k, default_config_for(batch, m, n, k, precision=self.precision), a16=a16)
+            entry = self.tune(batch, m, n, k, default_config_for(batch, m, n, k, precision=precision), a16=a16,
+                              precision=precision)
             if entry["candidates"]:
                 self._remember(key, entry)
         self.log.append({"shape": (batch, m, n, k), "source": source, **({"a16": True} if a16 else {}), **entry})
         return dict(entry["config"])
 
     # the lowering may pass a16 (a user's fn(graph, kernel) gets two arguments)
-    config_for.accepts_a16 = True
+    config_for.accepts_a16 = config_for.accepts_f16 = True
 
-    def _build(self, config, batch, m, n, k, weight, bias, a16=False):
+    def _build(self, config, batch, m, n, k, weight, bias, a16=False, precision=None):
         from kiln.api import Options, compile_graph
 
-        options = Options(device="cuda", cuda_graphs=False, matmul_precision=self.precision,
+        precision = precision or self.precision
+        options = Options(device="cuda", cuda_graphs=False, matmul_precision="fp32" if precision == "f16x3" else precision,
                           gpu_matmul_config=lambda *_: dict(config))
         exe, _ = compile_graph(_linear_graph(batch, m, n, k, weight, bias, a16), options)
         return exe
 
-    def _trials(self, batch, m, n, k, configs, a16=False):
+    def _trials(self, batch, m, n, k, configs, a16=False, precision=None):
         """Build every configuration and keep those whose result matches
         float64; returns (trials, reasons for the rejected ones)."""
         import torch
@@ -511,12 +550,15 @@ class GPUAutotuner:
             a = (a - a.mean(-1, keepdim=True)) / (a.var(-1, unbiased=False, keepdim=True) + LN_EPS).sqrt()
         exact = a @ w.double() + bias.double()
         scale = float(exact.abs().max()) or 1.0
-        tolerance = 1e-4 if self.precision == "fp32" else 2e-2
+        precision = precision or self.precision
+        tolerance = 1e-4 if precision in ("fp32", "f16x3") else 2e-2
         x_dev = x.to(device())
         trials, rejected = [], []
         for config in configs:
             try:
-                exe = self._build(config, batch, m, n, k, w.numpy(), bias.numpy(), a16)
+                exe = self._build(config, batch, m, n, k, w.numpy(), bias.numpy(), a16, precision)
+                if precision == "f16x3" and not any(f"tile {config['tile']} " in l.summary for l in exe.program.launches):
+                    raise RuntimeError("the plan keeps this product off fp16 pairs")
                 (out,) = exe(x_dev)
                 err = float((out.double().cpu() - exact).abs().max()) / scale
             except Exception as failure:  # noqa: BLE001 - a candidate that fails is dropped, never fatal
@@ -529,10 +571,13 @@ class GPUAutotuner:
                 rejected.append(f"{config}: relative error {err:.1e}")
         return trials, rejected
 
-    def tune(self, batch, m, n, k, default, a16=False):
+    def tune(self, batch, m, n, k, default, a16=False, precision=None):
         started = time.perf_counter()
-        configs = [default] + [c for c in candidates(batch, m, n, k, precision=self.precision) if c != default]
-        trials, rejected = self._trials(batch, m, n, k, configs, a16)
+        precision = precision or self.precision
+        # (fp16 pairs: the product reads a LayerNorm's output, stored as pairs)
+        a16 = a16 or precision == "f16x3"
+        configs = [default] + [c for c in candidates(batch, m, n, k, precision=precision) if c != default]
+        trials, rejected = self._trials(batch, m, n, k, configs, a16, precision)
         if not trials:
             warnings.warn(f"Kiln: no GEMM config passed for {batch}x{m}x{n}x{k}; keeping the default. "
                           + "; ".join(rejected[:3]))

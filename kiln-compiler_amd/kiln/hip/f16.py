@@ -1,0 +1,78 @@
+"""fp16-pair copies of GEMM weights (fp32 products on the fp16 matrix cores).
+
+A value x is held as h = fp16(x * 2^e) and l = fp16(x * 2^e - h): 23 of its 24
+significant bits (csrc/kh_common.hpp). The library reads B as [batch][N][K']
+rows (K' = K rounded up to 8, zero padded), in blocks of 8 values: 16 bytes of
+h, then 16 bytes of l. Each output column n has its own power of two, which
+puts the column's largest weight just below 2^15; the product's epilogue
+multiplies by ``column_scales``, one exact power of two per column that takes
+back the weights' scale and the activations'.
+"""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+# the largest scaled magnitude is below 2^TOP: fp16's largest finite value is
+# 65504, and a bound on activations may be missed by rounding
+TOP = 14
+# exponents that keep every scale and product of scales a normal float32
+WEIGHT_EXPONENTS = (-80, 80)
+ACTIVATION_EXPONENTS = (-40, 40)
+
+
+def activation_exponent(bound: float):
+    """e with bound * 2^e <= 2^TOP for activations of magnitude <= bound, or
+    None when the bound is no use (not finite, or its scale out of range)."""
+    if not math.isfinite(bound) or bound <= 0.0:
+        return None
+    e = TOP - math.ceil(math.log2(bound))
+    low, high = ACTIVATION_EXPONENTS
+    return e if low <= e <= high else None
+
+
+def padded_k(k: int) -> int:
+    return (k + 7) // 8 * 8
+
+
+def _rows(data: np.ndarray, offset: int, strides, batch: int, k: int, n: int) -> torch.Tensor:
+    """The [batch, K, N] view (element offset, strides over (b, k, n)) of a
+    constant as float32 [batch, N, K] (a view)."""
+    flat = torch.from_numpy(np.ascontiguousarray(data, dtype=np.float32).reshape(-1))
+    sb, sk, sn = (int(s) for s in strides)
+    return torch.as_strided(flat, (batch, n, k), (sb, sn, sk), offset)
+
+
+def row_exponents(data, offset, strides, batch: int, k: int, n: int) -> torch.Tensor:
+    """e [batch, N] (int32): a row's largest magnitude times 2^e lands in
+    [2^TOP, 2^(TOP + 1))."""
+    rows = _rows(data, offset, strides, batch, k, n)
+    top = torch.maximum(rows.amax(dim=-1), -rows.amin(dim=-1)) if k else torch.zeros(batch, n)
+    _, exponent = torch.frexp(top)   # top in [2^(exponent - 1), 2^exponent)
+    return torch.where(top > 0, TOP + 1 - exponent, torch.zeros_like(exponent)).clamp(*WEIGHT_EXPONENTS)
+
+
+def pair_rows(data, offset, strides, batch: int, k: int, n: int) -> np.ndarray:
+    """The [batch, N, K'] pair copy (int32 words) of the [batch, K, N] view of
+    a constant, each row times its own power of two (row_exponents)."""
+    e = row_exponents(data, offset, strides, batch, k, n)
+    rows = _rows(data, offset, strides, batch, k, n).contiguous()
+    rows = rows * torch.ldexp(torch.ones(()), e).unsqueeze(-1)
+    kp = padded_k(k)
+    if kp != k:
+        rows = torch.nn.functional.pad(rows, (0, kp - k))
+    rows = rows.view(batch, n, kp // 8, 8)
+    blocks = torch.empty(batch, n, kp // 8, 2, 8, dtype=torch.float16)
+    blocks[:, :, :, 0] = rows   # (rounds to nearest)
+    blocks[:, :, :, 1] = rows.sub_(blocks[:, :, :, 0])
+    return blocks.numpy().view(np.int32).reshape(batch, n, kp)
+
+
+def column_scales(data, offset, strides, batch: int, k: int, n: int, activation_e: int) -> np.ndarray:
+    """2^-(e + activation_e) per column (float32 [batch, N]): what a product of
+    the scaled operands is multiplied by."""
+    e = row_exponents(data, offset, strides, batch, k, n).numpy()
+    return np.ldexp(np.float32(1.0), -(e + activation_e)).astype(np.float32)

@@ -28,7 +28,8 @@ GEMV_PRO_NONE, GEMV_PRO_LAYERNORM, GEMV_PRO_ATTN = 0, 1, 2
 GEMV_CHAIN = 1   # KH_GEMV_CHAIN: kh_launch.variant flag of a GEMV launch
 ATTN_SCALE_NONE, ATTN_SCALE_MUL, ATTN_SCALE_DIV = 0, 1, 2
 ROW_GENERIC, ROW_LAYERNORM, ROW_SOFTMAX = 0, 1, 2
-PREC_FP32, PREC_BF16, PREC_BF16X3 = 0, 1, 2
+PREC_FP32, PREC_BF16, PREC_BF16X3, PREC_F16X3 = 0, 1, 2, 3
+PAIR_BF16, PAIR_F16 = 0, 1   # KH_PAIR_*: kh_launch.cfg[6] of a pair-storing ROW or ATTN launch
 NOALLOC_WORKSPACE_BYTES = 16 << 20   # KH_NOALLOC_WORKSPACE_BYTES: kh_plan_run_noalloc's device array
 
 OPCODES = ["mov", "add", "sub", "mul", "div", "max", "min", "neg", "relu", "exp", "tanh", "sigmoid",

@@ -29,8 +29,9 @@ import hashlib
 import math
 from dataclasses import dataclass, field
 
-from kiln.hip import autotune, bf16
+from kiln.hip import autotune, bf16, f16
 from kiln.hip import lib as kl
+from kiln.hip.bounds import Bounds
 from kiln.ir import ops
 from kiln.ir.core import Graph, Kernel
 from kiln.passes.buffers import Layout, compute_layouts, kernel_inputs, kernel_outputs
@@ -207,11 +208,14 @@ class _Lowerer:
         self.users = graph.users()
         self.bf16_buffers = set()   # arena buffers held as bf16 (plan_bf16_storage)
         self.pair_buffers = set()   # arena buffers held as pair words (plan_pair_storage)
+        self.f16_buffers = {}       # arena buffers held as fp16 pairs -> exponent of their scale (plan_f16_storage)
+        self.bounds = Bounds(graph, self._layer_norm_of, self._attention_value_of)
         self.precision = precision
         self.matmul_config = matmul_config
         self.program = Program(precision=precision)
         self.const_slot = {}
         self._cfg = {}
+        self._f16 = {}
         self.prologue = {}   # matmul kernel -> (x, gamma, beta, fparams, x as [rows, K]) of a fused LayerNorm
         self.attn_prologue = {}  # GEMV kernel -> (attention match, strides, mask mode, (heads, tk, dh))
 
@@ -248,6 +252,12 @@ class _Lowerer:
         """Is v's storage an arena buffer held as pair words (see plan_pair_storage)?"""
         lay = self.layouts.get(v)
         return lay is not None and lay.base[0] == "arena" and lay.base[1] in self.pair_buffers
+
+    def stored_f16(self, v):
+        """Exponent of the scale of v's storage as fp16 pairs, or None when v
+        is not stored that way (see plan_f16_storage)."""
+        lay = self.layouts.get(v)
+        return self.f16_buffers.get(lay.base[1]) if lay is not None and lay.base[0] == "arena" else None
 
     def as_bf16(self, r, v):
         """Ref r of v re-expressed over v's bf16 storage: the offset in bf16
@@ -381,6 +391,113 @@ class _Lowerer:
         if prec != "bf16x3" or (tile not in autotune.K_CONTIGUOUS | autotune.SMALL_M and int(cfg.get("splitk", 1)) > 1):
             return False
         return self._bias_act_epilogue(k, buf)
+
+    def plan_f16_storage(self):
+        """fp32 plans: the A operand of every product on fp16 pairs is stored
+        that way by its producer (matmul_choice gives such a configuration only
+        where it can be): {arena buffer: exponent of its scale}."""
+        out = {}
+        if self.precision != "fp32":
+            return out
+        for k in self.g.kernels:
+            if k.kind == "matmul" and k not in self.prologue and self.matmul_choice(k)[1] == "f16x3":
+                buf, e = self.f16_operand(k)
+                out[buf] = e
+        return out
+
+    def f16_operand(self, k):
+        """(arena buffer, exponent of its scale) of matmul kernel k's A operand
+        if k can run on fp16 pairs: B a constant, K whole 32-deep steps, A a
+        whole buffer with unit K stride and rows of whole 32-byte blocks, bounded
+        (kiln/hip/bounds.py), read by k alone, not a graph result, and written
+        by a launch that can store fp16 pairs. Otherwise None."""
+        if k not in self._f16:
+            self._f16[k] = self._f16_operand(k)
+        return self._f16[k]
+
+    def _f16_operand(self, k):
+        if self.precision != "fp32" or k.kind != "matmul" or k in self.prologue:
+            return None
+        mm = next(n for n in k.nodes if n.op == "matmul")
+        a, b = mm.inputs
+        if a.shape[-2] <= 1 or a.shape[-1] % 32 or a.shape[-1] == 0 or not self.skinny_ok(mm):
+            return None
+        lay = self.layouts[a]
+        if lay.base[0] != "arena" or lay.offset != 0 or any(
+                st % 8 for st, ext in zip(lay.strides[:-1], lay.shape[:-1]) if ext > 1):
+            return None
+        buf = lay.base[1]
+        if buf.type.nbytes != 4 * math.prod(a.shape) or self._arena_readers().get(buf) != {k} or buf in self.g.results:
+            return None
+        producer = self.g.kernel_of(buf.node)
+        if producer is None or not self._writes_f16(producer, buf):
+            return None
+        e = f16.activation_exponent(self.bounds.largest(a))
+        if e is None or not math.isfinite(self.bounds._column_norm(b)):
+            return None
+        return buf, e
+
+    def _writes_f16(self, k, buf) -> bool:
+        """Can kernel k write its output `buf` as fp16 pairs? The one-wave
+        LayerNorm, the blocked attention kernels, and a product with a bias
+        [+ GELU / ReLU] epilogue that runs on fp16 pairs itself or on an fp32
+        small-M configuration."""
+        if k.kind in ("attention", "reduction"):
+            if k.kind == "attention":
+                from kiln.hip.attention import match_kernel
+
+                m = match_kernel(self.g, k)
+                if m is None or any(st % 8 for st in self.layouts[m.result].strides[:-1]):
+                    return False
+            return (buf.shape[-1] % 8 == 0 and self._rounds_to_bf16(k, buf, precision="f16x3")
+                    and (k.kind == "attention" or self._one_wave_rows(k, buf)))
+        if k.kind != "matmul" or self.is_gemv(k) or buf.shape[-1] % 8 or kernel_outputs(self.g, k, self.users) != [buf]:
+            return False
+        cfg, prec = self.matmul_choice(k)
+        small = prec == "fp32" and int(cfg.get("tile", -1)) in autotune.SMALL_M
+        return (prec == "f16x3" or small) and self._bias_act_epilogue(k, buf)
+
+    def _layer_norm_of(self, k, v):
+        """(factor of the variance's sum, gamma, beta) if v is the output of a
+        LayerNorm kernel k, else None."""
+        reds = [n for n in k.nodes if n.op.startswith("reduce_")]
+        outs = kernel_outputs(self.g, k, self.users)
+        if outs != [v] or not reds or not all(is_row_reduction(n) for n in reds):
+            return None
+        variant, fparams, (has_g, has_b), ordered = self._row_pattern(k, reds, outs, self._externals(k))
+        if variant != kl.ROW_LAYERNORM or ordered is None:
+            return None
+        return fparams[1], ordered[1] if has_g else None, ordered[1 + has_g] if has_b else None
+
+    def _one_wave_rows(self, k, buf) -> bool:
+        """Does LayerNorm kernel k (out buf) meet the library's conditions for
+        the one-wave kernel: rows at one stride, all operands in aligned
+        16-byte pieces?"""
+        _, _, _, ordered = self._row_pattern(k, [n for n in k.nodes if n.op.startswith("reduce_")], [buf],
+                                             self._externals(k))
+        if ordered is None or not math.prod(buf.shape):
+            return False
+        x = self._rows_layout(ordered[0], (math.prod(buf.shape[:-1]), buf.shape[-1]))
+        if x is None or x.strides[-1] != 1 or x.offset % 4 or x.strides[0] % 4:
+            return False
+        lays = [self.layouts.get(p) for p in ordered[1:]]
+        return all(lay is not None and lay.strides[-1] == 1 and lay.offset % 4 == 0 for lay in lays)
+
+    def _externals(self, k):
+        members = set(k.nodes)
+        out = []
+        for n in k.nodes:
+            for v in n.inputs:
+                if (v.node not in members or v.node is None) and not self.is_imm(v) and v not in out:
+                    out.append(v)
+        return out
+
+    def _attention_value_of(self, k, v):
+        """The V operand of attention kernel k if v is its result, else None."""
+        from kiln.hip.attention import match_kernel
+
+        m = match_kernel(self.g, k)
+        return m.v if m is not None and (v is m.result or v in kernel_outputs(self.g, k, self.users)) else None
 
     def _bias_act_epilogue(self, k, buf) -> bool:
         """Is matmul kernel k's tape out = act(acc + bias), act none, GELU or
@@ -748,6 +865,10 @@ class _Lowerer:
         self._check_refs(refs)
 
         d = self.new_desc(kl.FAM_ROW, "row", k, shape)
+        f16_out = [v for v in outs if self.stored_f16(v) is not None]
+        for v in f16_out:
+            bf16_mask |= 1 << (16 + out_ref[v])
+            d.cfg[6], d.fparams[3] = kl.PAIR_F16, 2.0 ** self.stored_f16(v)
         d.cfg[7] = bf16_mask
         for j, r in enumerate(refs):
             d.refs[j] = r
@@ -851,7 +972,7 @@ class _Lowerer:
             kind += " out:bf16"
             nbytes -= 2 * sum(math.prod(v.shape) for v in outs)
         if bf16_mask >> 16:
-            kind += " out:pairs"
+            kind += " out:f16" if f16_out else " out:pairs"
         self.add(d, k, f"{kind} rows {list(rows)} x {inner}, {len(t.segments)} passes"
                        f"{'' if single else ' (chunked)'}: {' '.join(n.op for n in k.nodes)}", nbytes=nbytes)
 
@@ -952,12 +1073,18 @@ class _Lowerer:
             d.cfg[7] |= 1
         if not pro and not gemv and self.stored_pairs(a):
             d.cfg[7] |= 1 << 16
+        on_f16 = prec == "f16x3"
+        if on_f16:
+            d.cfg[7] |= 1 << 16
+            d.fparams[0] = 2.0 ** self.stored_f16(a)
         k_major = not gemv and int(cfg.get("tile", -1)) in autotune.NK_B
         nk = (gemv and self.layouts[b].base[0] == "const" and kk % 4 == 0) or k_major
-        derived_b = prec in ("bf16", "bf16x3") or nk
+        derived_b = prec in ("bf16", "bf16x3", "f16x3") or nk
         d.refs[1] = b_ref = ref3(b, (batch, kk, n), register=not derived_b)
         if prec in ("bf16", "bf16x3"):
             d.refs[1] = self.bf16_weight(b, d.refs[1], batch, kk, n, split=prec == "bf16x3")
+        elif on_f16:
+            d.refs[1], column_scales = self.f16_weight(b, b_ref, batch, kk, n, self.stored_f16(a))
         elif nk:
             d.refs[1] = self.nk_weight(b, b_ref, batch, kk, n, scale=pro[1] if pro and not gemv else None)
         externals = []
@@ -981,8 +1108,14 @@ class _Lowerer:
                 d.cfg[7] |= 1 << (2 + out_ref[v])
             if self.stored_pairs(v):
                 d.cfg[7] |= 1 << (16 + 2 + out_ref[v])
+            if self.stored_f16(v) is not None:
+                d.cfg[7] |= 1 << (16 + 2 + out_ref[v])
+                d.fparams[3] = 2.0 ** self.stored_f16(v)
             refs.append(r)
         pro_refs = []
+        if on_f16:
+            d.cfg[5] = 2 + len(refs)
+            pro_refs.append(column_scales)
         attn_work = None
         if gemv and k in self.attn_prologue:
             pro_refs, *attn_work = self.attn_prologue_refs(d, k, 2 + len(refs))
@@ -1044,7 +1177,8 @@ class _Lowerer:
                    "precision": cfg.get("precision", self.precision)}
         d.cfg[1] = int(cfg.get("tile", 0))
         d.cfg[2] = int(cfg.get("splitk", 1))
-        d.cfg[3] = {"fp32": kl.PREC_FP32, "bf16": kl.PREC_BF16, "bf16x3": kl.PREC_BF16X3}[prec]
+        d.cfg[3] = {"fp32": kl.PREC_FP32, "bf16": kl.PREC_BF16, "bf16x3": kl.PREC_BF16X3,
+                    "f16x3": kl.PREC_F16X3}[prec]
         flops = 2 * batch * m * n * kk
         nbytes = 4 * (math.prod(a.shape) + math.prod(b.shape) + sum(math.prod(v.shape) for v in externals)
                       + len(outs) * math.prod(out_shape))
@@ -1065,6 +1199,8 @@ class _Lowerer:
             summary += " A:pairs"
         if any(self.stored_pairs(v) for v in outs):
             summary += " out:pairs"
+        if any(self.stored_f16(v) is not None for v in outs):
+            summary += " out:f16"
         if pro:
             summary += " prologue: layernorm"
             nbytes += 4 * kk * len(pro_refs)
@@ -1096,12 +1232,22 @@ class _Lowerer:
         """(configuration, precision) of matmul kernel k, asked once per kernel."""
         if k not in self._cfg:
             mm = next(n for n in k.nodes if n.op == "matmul")
+            asks_f16 = getattr(self.matmul_config, "accepts_f16", False)
+            if asks_f16 and self._prefers_f16(k):
+                self._cfg[k] = (dict(self.matmul_config(self.g, k, f16=True)), "f16x3")
+                return self._cfg[k]
             if getattr(self.matmul_config, "accepts_a16", False) and (
                     self.a16_buffer(k) is not None or self.a_pair_buffer(k, check_choice=False) is not None):
                 # the tuner times this product reading A as bf16 / pair words, as the plan can store it
                 cfg = dict(self.matmul_config(self.g, k, a16=True))
             else:
                 cfg = dict(self.matmul_config(self.g, k))
+            if autotune.PRECISION.get(int(cfg.get("tile", -1))) == "f16x3" and self.f16_operand(k) is not None:
+                # a caller's configuration on fp16 pairs, where the product can run on them
+                m, kk = mm.inputs[0].shape[-2:]
+                if autotune.k_major_fits(m, kk, int(cfg["tile"])):
+                    self._cfg[k] = (cfg, "f16x3")
+                    return self._cfg[k]
             prec = cfg.get("precision", self.precision)
             if prec in ("bf16", "bf16x3") and self.layouts[mm.inputs[1]].base[0] != "const":
                 # bf16 inputs need B as a build-time bf16 copy of a constant; a
@@ -1122,6 +1268,21 @@ class _Lowerer:
                 cfg = autotune.default_config_for(batch, m, n, kk, precision=prec, skinny=False)
             self._cfg[k] = (cfg, prec)
         return self._cfg[k]
+
+    def _prefers_f16(self, k) -> bool:
+        """Does matmul kernel k (an fp32 product) run on fp16 pairs? Wherever it
+        can, except where it would take a LayerNorm as its prologue: that
+        saves a launch, and stays on the fp32 small-M kernel."""
+        operand = self.f16_operand(k)
+        if operand is None:
+            return False
+        m, kk = next(n for n in k.nodes if n.op == "matmul").inputs[0].shape[-2:]
+        producer = self.g.kernel_of(operand[0].node)
+        if m > LN_PROLOGUE_MAX_ROWS or kk > 1024 or producer.kind != "reduction":
+            return True
+        tile = int(self.matmul_config(self.g, k).get("tile", -1))
+        bm, wk = autotune.TILES[tile][0], autotune.TILES[tile][5]
+        return not (tile in autotune.SMALL_M and bm % wk == 0 and bm <= 4 * wk)
 
     def skinny_ok(self, mm) -> bool:
         """The skinny-M and K-contiguous GEMMs read B as a build-time
@@ -1395,6 +1556,26 @@ class _Lowerer:
         pairs = 1 if mode == kl.ATTN_MASK_CAUSAL else tk
         return refs, 4 * heads * pairs * dh, 4 * heads * dh * (2 + 2 * tk)
 
+    def f16_weight(self, b, ref, batch, kk, n, activation_e):
+        """Refs of the fp16-pair [batch][N][K'] copy of constant view `b`
+        (fp32 ref `ref` over (b, k, n)) and of the powers of two that take back
+        its columns' scales and the activations' (2^activation_e); both are
+        derived constants, made when the executable is built."""
+        src = self.layouts[b].base[1]
+        strides = (int(ref.strides[0]), int(ref.strides[1]), int(ref.strides[2]))
+        at = f"{int(ref.offset)}:{strides[0]},{strides[1]},{strides[2]}:{batch}x{kk}x{n}"
+        weight, scales = f"{src}@f16:{at}", f"{src}@f16s:{at}:{activation_e}"
+        recipe = (src, int(ref.offset), strides, batch, kk, n)
+        self.program.derived[weight] = recipe
+        self.program.derived[scales] = recipe + (("", int(activation_e), 0),)
+        row = f16.padded_k(kk)
+        r, c = kl.Ref(), kl.Ref()
+        r.base, r.index = self.slot_of(("const", weight))
+        r.strides[0], r.strides[1], r.strides[2] = (n * row if batch > 1 else 0), 1, row
+        c.base, c.index = self.slot_of(("const", scales))
+        c.strides[0], c.strides[1], c.strides[2] = (n if batch > 1 else 0), 0, 1
+        return r, c
+
     def bf16_weight(self, b, ref, batch, kk, n, split=False):
         """Ref of the bf16 [batch][N][K'] copy of constant view `b` (whose fp32
         ref over (b, k, n) is `ref`), or with `split` the three-pass
@@ -1436,6 +1617,9 @@ class _Lowerer:
                 d.cfg[7] |= 1 << j
             if self.stored_pairs(v):  # (pair words: addressed as fp32)
                 d.cfg[7] |= 1 << (16 + j)
+            if self.stored_f16(v) is not None:   # the output
+                d.cfg[7] |= 1 << (16 + j)
+                d.cfg[6], d.fparams[3] = kl.PAIR_F16, 2.0 ** self.stored_f16(v)
             d.refs[j] = r
         d.n_refs = 4
         mode = kl.ATTN_MASK_NONE
@@ -1478,7 +1662,7 @@ class _Lowerer:
         if d.cfg[7] >> 16 & 7:
             scale += ", qkv:pairs"
         if d.cfg[7] >> 16 & 8:
-            scale += ", out:pairs"
+            scale += ", out:f16" if d.cfg[6] == kl.PAIR_F16 else ", out:pairs"
         self.add(d, k, f"{batch} heads x {tq} queries x {tk} keys, head dim {dh}, {what}{scale}",
                  flops=flops, nbytes=nbytes)
 
@@ -1492,6 +1676,7 @@ class _Lowerer:
         fused = self.find_ln_prologues() | self.find_attn_prologues()
         self.bf16_buffers = self.plan_bf16_storage()
         self.pair_buffers = self.plan_pair_storage()
+        self.f16_buffers = self.plan_f16_storage()
         for k in self.g.kernels:
             if k in fused:
                 continue
@@ -1515,6 +1700,18 @@ class _Lowerer:
                                                    live[0], live[-1]))
         self.program.arena_buffers.sort(key=lambda b: b[1])
         return self.program
+
+
+def operand_scales(graph: Graph) -> str:
+    """The exponents that fp16 pairs could scale the graph's products by: what
+    an fp32 plan depends on of the constants' values."""
+    low = _Lowerer(graph, "fp32", None)
+    out = []
+    for k in graph.kernels:
+        if k.kind == "matmul":
+            mm = next(n for n in k.nodes if n.op == "matmul")
+            out.append(f16.activation_exponent(low.bounds.largest(mm.inputs[0])))
+    return repr(out)
 
 
 def lower_graph(graph: Graph, precision: str = "fp32", matmul_config=None, gemv_chains: bool = False) -> Program:

@@ -22,7 +22,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from kiln.hip import bf16
+from kiln.hip import bf16, f16
 from kiln.hip import lib as kl
 
 MiB = 2**20
@@ -106,10 +106,9 @@ def nk_copy(data: np.ndarray, offset: int, strides, batch: int, k: int, n: int) 
     [batch, K, N] view (element offset, strides over (b, k, n)) of a constant:
     the layout of the K-contiguous GEMV kernel."""
     flat = np.ascontiguousarray(data, dtype=np.float32).reshape(-1)
-    sb, sk, sn = (int(s) for s in strides)
-    idx = (offset + np.arange(batch)[:, None, None] * sb + np.arange(n)[None, :, None] * sn
-           + np.arange(k)[None, None, :] * sk)
-    return np.ascontiguousarray(flat[idx])
+    sb, sk, sn = (int(s) * flat.itemsize for s in strides)
+    view = np.lib.stride_tricks.as_strided(flat[offset:], (batch, n, k), (sb, sn, sk), writeable=False)
+    return np.ascontiguousarray(view)
 
 
 def host_constant(program, constants: dict, name: str) -> np.ndarray:
@@ -119,6 +118,9 @@ def host_constant(program, constants: dict, name: str) -> np.ndarray:
     if recipe is None:
         return np.ascontiguousarray(constants[name], np.float32)
     src, offset, strides, batch, k, n = recipe[:6]
+    if "@f16:" in name or "@f16s:" in name:
+        args = (constants[src], offset, strides, batch, k, n)
+        return f16.pair_rows(*args) if "@f16:" in name else f16.column_scales(*args, recipe[6][1])
     if "@nk:" in name:
         return nk_copy(constants[src], offset, strides, batch, k, n)
     if "@nkg:" in name or "@lnc:" in name or "@lng:" in name:

@@ -55,14 +55,15 @@ def warm_up(seconds=1.0):
 def main(argv=None):
     p = argparse.ArgumentParser(description=__doc__.splitlines()[0])
     p.add_argument("--out", default=str(autotune.SHIPPED_PATH))
-    p.add_argument("--precision", nargs="+", choices=("fp32", "bf16", "bf16+a16", "bf16x3", "bf16x3+a16"), default=None,
+    p.add_argument("--precision", nargs="+", default=None,
+                   choices=("fp32", "f16x3", "bf16", "bf16+a16", "bf16x3", "bf16x3+a16"),
                    help="re-tune only these precisions and keep the table's other entries")
     p.add_argument("--max-m", type=int, default=None,
                    help="re-tune only shapes with at most this many rows and keep the table's other entries")
     args = p.parse_args(argv)
     warm_up()
     shapes = [s for s in SHAPES if args.max_m is None or s[0] <= args.max_m]
-    precisions = args.precision or ("fp32", "bf16", "bf16+a16", "bf16x3", "bf16x3+a16")
+    precisions = args.precision or ("fp32", "f16x3", "bf16", "bf16+a16", "bf16x3", "bf16x3+a16")
     table = {}
     if args.precision or args.max_m is not None:
         retuned = {(p_, f"1x{m}x{n}x{k}") for p_ in precisions for m, n, k in shapes}
@@ -71,12 +72,14 @@ def main(argv=None):
     for precision in precisions:
         a16 = precision.endswith("+a16")
         base = precision.split("+")[0]
-        tuner = autotune.GPUAutotuner(precision=base, use_cache=False, use_shipped=False)
+        f16 = base == "f16x3"   # the block's fp32 products on fp16 pairs
+        tuner = autotune.GPUAutotuner(precision="fp32" if f16 else base, use_cache=False, use_shipped=False)
         device = tuner.device_key()
         for m, n, k in shapes:
-            if a16 and (m, n, k) not in BLOCK:
+            if (a16 or f16) and (m, n, k) not in BLOCK:
                 continue
-            entry = tuner.tune(1, m, n, k, autotune.default_config_for(1, m, n, k, precision=base), a16=a16)
+            entry = tuner.tune(1, m, n, k, autotune.default_config_for(1, m, n, k, precision=base), a16=a16,
+                               precision=base)
             if entry["candidates"]:
                 table[f"{device}|{precision}|1x{m}x{n}x{k}"] = entry
             print(f"{precision} {m}x{n}x{k}: {entry['config']} {entry['tflops']} TFLOP/s", flush=True)

@@ -1,0 +1,156 @@
+"""fp32 products on fp16 pairs, on the CPU: the pair copies of weights, the
+bounds that make a fixed activation scale safe, which products take the path,
+and the plan's meaning through the host interpreter."""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import kiln
+import oracle
+from kiln.hip import autotune, f16
+from kiln.hip.bounds import Bounds
+from kiln.hip.lowering import _Lowerer, lower_graph, operand_scales
+from models.transformer import Block, gpt2_init_
+from test_interpret import check
+from test_lowering import lowered
+
+
+@pytest.fixture
+def interpreting(monkeypatch):
+    monkeypatch.setenv("KILN_HIP_INTERPRET", "1")
+
+
+def decode(copy, scales):
+    b, n, kp = copy.shape
+    h = copy.view(np.float16).reshape(b, n, kp // 8, 2, 8).astype(np.float64)
+    return (h[:, :, :, 0] + h[:, :, :, 1]).reshape(b, n, kp) * scales.astype(np.float64)[:, :, None]
+
+
+@pytest.mark.parametrize("k,n", [(8, 3), (40, 24), (61, 5), (768, 2)])
+def test_pair_copy_holds_23_bits_per_column(k, n):
+    # each column its own power of two: columns 2^-40 .. 2^30 in size keep the
+    # relative precision of their largest weights (half an ulp of l: 2^-23 of
+    # the value, 2^-25 of 2^-14 of the column's largest below that)
+    w = np.random.default_rng(0).standard_normal((k, n)).astype(np.float32)
+    w *= (2.0 ** np.linspace(-40, 30, n)).astype(np.float32)
+    if n > 3:
+        w[:, 3] = 0.0
+    args = (w, 0, (0, n, 1), 1, k, n)
+    got = decode(f16.pair_rows(*args), f16.column_scales(*args, 0))[0, :, :k].T
+    top = np.abs(w).max(axis=0)
+    assert (np.abs(got - w) <= 2.0 ** -23 * np.abs(w) + 2.0 ** -39 * top).all()
+    assert (f16.pair_rows(*args).reshape(n, -1)[:, f16.padded_k(k):] == 0).all()
+    assert np.array_equal(f16.column_scales(*args, 5), f16.column_scales(*args, 0) / 32)
+
+
+def _bounds(model, x):
+    g, _ = lowered(model, x, fuse_attention=True)
+    return g, _Lowerer(g, "fp32", None)
+
+
+@pytest.mark.parametrize("scale", [1e-6, 1.0, 1e6])
+def test_bounds_hold_whatever_the_input(scale):
+    # LayerNorm -> Linear -> GELU -> Linear: every product's A operand stays
+    # under its bound, for inputs of any size and rows with one outlier
+    torch.manual_seed(1)
+    ln, fc, proj = torch.nn.LayerNorm(64), torch.nn.Linear(64, 256), torch.nn.Linear(256, 64)
+    torch.nn.init.normal_(ln.weight, 1.0, 0.5), torch.nn.init.normal_(ln.bias)
+    model = torch.nn.Sequential(ln, fc, torch.nn.GELU(), proj).eval()
+    x = torch.randn(300, 64) * scale
+    x[7] = 0.0
+    x[7, 3] = 1e5 * scale
+    g, low = _bounds(model, x)
+    tops = [low.bounds.largest(next(n for n in k.nodes if n.op == "matmul").inputs[0]) for k in g.kernels
+            if k.kind == "matmul"]
+    with torch.no_grad():
+        a = ln(x)
+        b = F.gelu(fc(a))
+    assert len(tops) == 2 and float(a.abs().max()) <= tops[0] and float(b.abs().max()) <= tops[1]
+    assert float(ln(x).abs().max()) > tops[0] / 64   # not vacuous
+    for top in tops:
+        assert top * 2.0 ** f16.activation_exponent(top) <= 2.0 ** f16.TOP
+
+
+def test_bounds_refuse_what_has_none():
+    assert f16.activation_exponent(float("inf")) is None and f16.activation_exponent(0.0) is None
+    assert f16.activation_exponent(1e30) is None
+    # a graph input, and a LayerNorm with a non-finite parameter
+    g, low = _bounds(torch.nn.Linear(64, 64).eval(), torch.randn(300, 64))
+    assert low.bounds.largest(g.args[0]) == float("inf")
+    ln = torch.nn.LayerNorm(64)
+    with torch.no_grad():
+        ln.weight[3] = float("inf")
+    g, prog = lowered(torch.nn.Sequential(ln, torch.nn.Linear(64, 64)).eval(), torch.randn(300, 64))
+    assert not any("f16x3" in l.summary for l in prog.launches)
+
+
+def test_which_products_run_on_pairs():
+    g, prog = lowered(Block(768, 12, 512), torch.randn(512, 768), fuse_attention=True)
+    matmuls = [l for l in prog.launches if "matmul" in l.name]
+    assert len(matmuls) == 4 and all(" f16x3" in l.summary for l in matmuls)
+    assert "out:f16" in prog.launches[0].summary and "out:f16" in prog.launches[2].summary
+    # T = 128: the products with a LayerNorm prologue stay fp32
+    g, prog = lowered(Block(768, 12, 128), torch.randn(128, 768), fuse_attention=True)
+    for l in prog.launches:
+        if "matmul" in l.name:
+            assert ("f16x3" in l.summary) != ("prologue: layernorm" in l.summary)
+    # a graph input as A, and a LayerNorm output that is also a result
+    ln, lin = torch.nn.LayerNorm(64).eval(), torch.nn.Linear(64, 96).eval()
+    for fn in (lambda t: lin(t), lambda t: (lin(ln(t)), ln(t))):
+        g, prog = lowered(fn, torch.randn(300, 64))
+        assert not any("f16x3" in l.summary for l in prog.launches)
+
+
+def test_plan_key_follows_the_scales():
+    # the scales are the only thing a plan takes from constants' values
+    lin = torch.nn.Sequential(torch.nn.LayerNorm(64), torch.nn.Linear(64, 96)).eval()
+    x = torch.randn(300, 64)
+    g1, p1 = lowered(lin, x)
+    with torch.no_grad():
+        lin[0].weight.mul_(100.0)
+    g2, p2 = lowered(lin, x)
+    assert operand_scales(g1) != operand_scales(g2)
+    assert p1.launches[-1].desc.fparams[0] != p2.launches[-1].desc.fparams[0]
+
+
+@pytest.mark.parametrize("T", [40, 300])
+def test_interpreted_block(interpreting, T):
+    model = gpt2_init_(Block(64, 2, T), seed=0).eval()
+    x = torch.randn(T, 64)
+    c = kiln.compile(model, (x,), device="cuda")
+    assert any("f16x3" in l.summary for l in c._exe.program.launches)
+    ref = oracle.block(x.numpy(), {k: v.numpy() for k, v in model.state_dict().items()}, 2)
+    np.testing.assert_allclose(c(x).numpy(), ref, rtol=1e-4, atol=1e-5)
+
+
+def test_interpreted_batched_weights(interpreting):
+    class Batched(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.ln, self.w = torch.nn.LayerNorm(96), torch.nn.Parameter(torch.randn(3, 96, 50) * 0.1)
+
+        def forward(self, t):
+            return self.ln(t) @ self.w
+
+    c = check(Batched().eval(), torch.randn(3, 300, 96))
+    assert any("f16x3" in l.summary for l in c._exe.program.launches)
+
+
+def test_callers_configuration_on_pairs():
+    # a caller may name a pair configuration; where the product cannot run on
+    # pairs it is a configuration of another precision like any other
+    tile = 102
+    cfg = lambda *_: {"tile": tile, "splitk": 1}
+    ln, lin = torch.nn.LayerNorm(64).eval(), torch.nn.Linear(64, 96).eval()
+    from kiln.api import Options, build_passes
+    from kiln.passes.manager import PassManager
+    from test_gpu import imported
+
+    for fn, on_pairs in ((lambda t: lin(ln(t)), True), (lambda t: lin(t), False)):
+        g = imported(fn, (torch.randn(300, 64),))
+        PassManager(build_passes(Options())).run(g)
+        prog = lower_graph(g, matmul_config=cfg)
+        assert (f"tile {tile} splitk 1 f16x3" in prog.launches[-1].summary) == on_pairs
+    assert autotune.PRECISION[tile] == "f16x3"

@@ -1,0 +1,121 @@
+"""Parity of the fp32 products on fp16 pairs (tiles of precision "f16x3"):
+against float64 of the fp32 inputs at the fp32 suite's tolerance, and with an
+error no larger than an fp32 MFMA configuration's that sums K in one chain."""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import kiln
+import oracle
+from kiln.hip import autotune
+from models.transformer import Block, gpt2_init_
+from test_gpu import ATOL, RTOL
+
+pytestmark = pytest.mark.gpu
+
+TILES = [t for t in sorted(autotune.TILES) if autotune.PRECISION[t] == "f16x3"]
+FP32_CHAIN = 4   # the fp32 copy pipeline's 32x64 tile
+
+
+class _LnLinear(torch.nn.Module):
+    """LayerNorm -> Linear, then an epilogue: none, "res" (residual), an
+    activation, or "tape" (one that the direct epilogue does not have)."""
+
+    def __init__(self, k, n, epilogue):
+        super().__init__()
+        self.ln, self.lin, self.epilogue = torch.nn.LayerNorm(k), torch.nn.Linear(k, n), epilogue
+        with torch.no_grad():
+            self.lin.weight.normal_(0.0, 1.0 / k ** 0.5)
+            self.ln.weight.normal_(1.0, 0.3), self.ln.bias.normal_(0.0, 0.3)
+
+    def forward(self, x, r):
+        y = self.lin(self.ln(x))
+        if self.epilogue == "res":
+            return y + r
+        if self.epilogue == "tape":
+            return torch.tanh(y) * r
+        return F.gelu(y, approximate=self.epilogue) if self.epilogue in ("tanh", "none") else y
+
+
+def _run(model, args, tile):
+    c = kiln.compile(model, args, device="cuda", cuda_graphs=False,
+                     gpu_matmul_config=lambda *_: {"tile": tile, "splitk": 1})
+    return c, c(*args)
+
+
+# M and N around and between tile edges, K from one step to more than the ring
+# holds, odd and even step counts
+SHAPES = [(1100, 200, 32, "res"), (1030, 133, 64, "linear"), (1027, 8, 96, "tanh"), (1153, 452, 160, "none"),
+          (1061, 97, 768, "tape"), (1025, 384, 224, "res")]
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_every_pair_configuration(tile):
+    for m, n, k, epilogue in SHAPES:
+        if tile in autotune.SMALL_M:
+            m -= 1020     # 5 .. 133 rows
+        torch.manual_seed(m + n + k)
+        model = _LnLinear(k, n, epilogue).eval()
+        args = (torch.randn(m, k) * 3 + 1, torch.randn(m, n))
+        print(tile, m, n, k, epilogue, flush=True)
+        c, out = _run(model, args, tile)
+        assert f"tile {tile} splitk 1 f16x3" in c._exe.program.launches[-1].summary
+        _, plain = _run(model, args, FP32_CHAIN)
+        with torch.no_grad():
+            ref = model.double()(*(t.double() for t in args))
+        np.testing.assert_allclose(out.cpu().double().numpy(), ref.numpy(), rtol=RTOL, atol=ATOL)
+        err, err_plain = ((t.cpu().double() - ref).norm() / ref.norm() for t in (out, plain))
+        # (a few roundings at K = 32: the two agree to a factor)
+        assert err <= (1.1 if k > 96 else 1.5) * err_plain + 1e-9, (err, err_plain)
+        for _ in range(3):
+            assert torch.equal(c(*args), out)
+
+
+def test_columns_of_very_different_size_keep_their_precision():
+    torch.manual_seed(3)
+    model = _LnLinear(256, 96, "linear").eval()
+    with torch.no_grad():
+        model.lin.weight *= (10.0 ** torch.linspace(-8, 4, 96))[:, None]
+        model.lin.bias.zero_()
+    args = (torch.randn(300, 256), torch.randn(300, 96))
+    _, out = _run(model, args, 102)
+    with torch.no_grad():
+        ref = model.double()(*(t.double() for t in args))
+    err = (out.cpu().double() - ref).norm(dim=0) / ref.norm(dim=0)
+    assert float(err.max()) <= 5e-7     # 24 steps' roundings; a shared scale would lose the small columns
+
+
+@pytest.mark.parametrize("loc,scale", [(0.0, 1e-4), (100.0, 1.0), (0.0, 1e8)])
+def test_rows_of_any_size_and_non_finite_rows(loc, scale):
+    torch.manual_seed(4)
+    model = _LnLinear(128, 200, "linear").eval()
+    x = torch.randn(300, 128) * scale + loc
+    bad = [3, 64, 299]
+    for row, v in zip(bad, (float("nan"), float("inf"), -float("inf"))):
+        x[row, 5] = v
+    args = (x, torch.randn(300, 200))
+    _, out = _run(model, args, 103)
+    _, plain = _run(model, args, FP32_CHAIN)
+    good = [i for i in range(300) if i not in bad]
+    assert torch.isnan(out[bad]).all()
+    # against the fp32 product on the same LayerNorm rows
+    np.testing.assert_allclose(out[good].cpu().numpy(), plain[good].cpu().numpy(), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("T", [16, 300, 777])
+def test_block_on_pairs(T):
+    model = gpt2_init_(Block(256, 4, T), seed=0).eval()
+    x = torch.randn(T, 256)
+    c = kiln.compile(model, (x,), device="cuda")
+    assert any("f16x3" in l.summary for l in c._exe.program.launches)
+    ref = oracle.block(x.numpy(), {k: v.numpy() for k, v in model.state_dict().items()}, 4)
+    np.testing.assert_allclose(c(x.cuda()).cpu().numpy(), ref, rtol=RTOL, atol=ATOL)
+    exe = c._exe
+    for _ in range(3):     # graph replays, with eager work between them
+        exe.replay_only()
+        torch.zeros(8, device="cuda").add_(1)
+    exe._static[0][0].copy_(x.cuda())
+    exe.replay_only()
+    assert torch.equal(exe._static[1][0], c(x.cuda()))
