@@ -188,7 +188,9 @@ typedef struct kh_pass {
  *        fp32); 2 three-pass bf16 (each of those inputs split into hi =
  *        bf16(x) and lo = bf16(x - hi), lo 0 for a non-finite hi, a product
  *        taken as lo.hi + hi.lo + hi.hi; fp32 q, k, v and 32 queries per
- *        workgroup).
+ *        workgroup); 3 fp16 pairs (q, k and v all stored that way, see below;
+ *        fparams[1] = 1 / (scale of q * scale of k), fparams[2] = 1 / scale
+ *        of v; 32 queries per workgroup).
  * cfg[] holds the family configuration (GEMM: tile id, split-K, precision).
  * bf16 storage (ROW, ATTN, GEMM): bit j of cfg[7] says refs[j] holds bf16
  * values (round to nearest even), its offset and strides counted in bf16
@@ -208,7 +210,7 @@ typedef struct kh_pass {
  * three-pass products (cfg[5] = 2), its q, k, v together, and on the
  * three-pass GEMM configurations the A operand (bit 16) and the output of a
  * direct epilogue without split-K.
- * fp16 pairs: an fp32 product on KH_PREC_F16X3 configurations (101-109) reads
+ * fp16 pairs: an fp32 product on KH_PREC_F16X3 configurations (101-110) reads
  * A and B as fp16 pairs: each value, scaled by a power of two into fp16's
  * range, as h = fp16(x) and l = fp16(x - h), a row in blocks of 8 values (16
  * bytes of h, then 16 bytes of l), 4 bytes a value, strides and offsets

@@ -50,6 +50,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "kh_attn_args.hpp"
 #include "kh_common.hpp"
 #include "kh_internal.hpp"
 
@@ -59,33 +60,6 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int kQB = 32;  // queries per workgroup
-constexpr int kKB = 32;  // keys per block
-// buffer resource word 3 for gfx9-family raw buffers: 32-bit data format
-constexpr int kBufferFlags = 0x00020000;
-
-struct AttnArgs {
-  const float *q, *k, *v;
-  float *o;                // (a bf16 array when o16)
-  const float *mask;
-  int64_t q_b, q_t, k_b, k_t, v_b, v_t, o_b, o_t, m_b, m_q, m_k;
-  int32_t batch, tq, tk, n_qblocks;
-  int32_t mask_mode, scale_mode;
-  float scale;
-  int32_t o16;             // the output is bf16 (its consumer is a bf16 matmul)
-  int32_t o_pair;          // the output is bf16 pair words (1) or fp16 pairs (2), as its consumer reads it
-  float o_scale;           // fp16 pairs: the power of two the output is scaled by
-  uint64_t *rec;           // timeline probe only: 8 words per wave (kh_probe_attn_timeline)
-};
-
-// Exchange between the two lane halves (lanes l and l ^ 32): returns
-// (x[l & 31], x[32 + (l & 31)]), the low half's value first in every lane,
-// so a combine of the two is the same in both halves. One v_permlane32_swap.
-__device__ __forceinline__ float2 halves(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 
 // BF: bf16 products (plans whose matrix products take bf16 inputs): Q and K
 // rounded to bf16 (round to nearest even) for the scores, the probabilities
@@ -929,6 +903,7 @@ class AttnOp final : public Op {
   bool in16 = false;  // q, k, v stored as bf16 (attn_kernel<..., BF, ..., IN16>)
   bool x3 = false;    // three-pass bf16 products (attn_kernel<..., BF, ..., X3>)
   bool p3 = false;    // q, k, v stored as pair words (attn_kernel<..., X3, P3>)
+  bool f16 = false;   // q, k, v stored as fp16 pairs (attn_f16_kernel)
   dim3 grid;
 
   hipError_t launch(float *const *ptrs, float *, hipStream_t stream) override {
@@ -938,6 +913,7 @@ class AttnOp final : public Op {
     for (int j = 0; j < 4; ++j)
       if (reinterpret_cast<uintptr_t>(ptrs[j]) & (j == 3 && a.o16 ? 7 : 15)) return hipErrorInvalidValue;
     if (a.batch == 0 || a.tq == 0) return hipSuccess;
+    if (f16) return launch_attn_f16(a, dh, nw, grid, stream);
     if (rows) {
       const dim3 g((unsigned)((a.batch * a.tq + 3) / 4));
       const bool add = a.mask_mode == KH_ATTN_MASK_ADD;
@@ -1083,12 +1059,13 @@ std::unique_ptr<Op> make_attn(const kh_launch &L, std::string &err, bool &unsupp
   // (attn_kernel<..., BF> or, for 16 queries per workgroup, attnbf_kernel),
   // 2 three-pass bf16 (attn_kernel<..., BF, ..., X3>, 32 queries per workgroup)
   const int prec = L.cfg[5];
-  if (prec < 0 || prec > 2) {
-    err = "attention: products precision must be 0 (fp32), 1 (bf16) or 2 (three-pass bf16)";
+  if (prec < 0 || prec > 3) {
+    err = "attention: products precision must be 0 (fp32), 1 (bf16), 2 (three-pass bf16) or 3 (fp16 pairs)";
     return nullptr;
   }
-  op->bf = prec >= 1;
+  op->bf = prec == 1 || prec == 2;
   op->x3 = prec == 2;
+  op->f16 = prec == 3;
   // 16 when 32-query blocks would give under 1.5 workgroups per CU (measured
   // on the GPT-2 block, 12 heads causal: T = 128 6.2 -> 4.7 us, 512 13.5 ->
   // 11.4 us; from T = 1024 on the 32-query kernel is faster); with bf16
@@ -1110,13 +1087,26 @@ std::unique_ptr<Op> make_attn(const kh_launch &L, std::string &err, bool &unsupp
   // pair words (cfg[7] bits 16 + j): q, k, v together (three-pass products)
   // and / or the output of a blocked kernel
   const uint32_t mp = pair_refs(L);
-  op->p3 = (mp & 7u) != 0;
+  op->p3 = (mp & 7u) != 0 && !op->f16;
+  if (op->f16) {
+    // fp16 pairs: q, k and v all stored that way, rows of whole 32-byte blocks
+    bool ok = (mp & 7u) == 7u && !m16 && qpw != 16 && pow2_scale(L.fparams[1]) && pow2_scale(L.fparams[2]);
+    for (int j = 0; j < 3; ++j)
+      ok = ok && L.refs[j].strides[0] % 8 == 0 && L.refs[j].strides[1] % 8 == 0 && L.refs[j].offset % 8 == 0;
+    if (!ok || ((mp >> 3 & 1) && L.cfg[6] != KH_PAIR_F16)) {
+      unsupported = true;
+      err = "attention: fp16 pairs need q, k and v in pair storage with rows of whole 32-byte blocks, "
+            "power-of-two scales, 32 queries per workgroup and an fp32 or fp16-pair output";
+      return nullptr;
+    }
+    a.qk_inv = L.fparams[1], a.v_inv = L.fparams[2];
+  }
   if ((mp & ~0xFu) || (op->p3 && ((mp & 7u) != 7u || !op->x3)) || (mp & m16)) {
     unsupported = true;
     err = "attention: pair storage of q, k, v needs all three and three-pass products; of the output, fp32 storage";
     return nullptr;
   }
-  op->q16 = !op->in16 && !op->x3 && (qpw == 16 || (qpw == 0 && (op->bf ? 2 * groups32 < current_device().cus
+  op->q16 = !op->in16 && !op->x3 && !op->f16 && (qpw == 16 || (qpw == 0 && (op->bf ? 2 * groups32 < current_device().cus
                                                               : 2 * groups32 < 3ll * current_device().cus)));
   a.n_qblocks = (int)((tq + (op->q16 ? 16 : kQB) - 1) / (op->q16 ? 16 : kQB));
   op->dh = (int)dh;
@@ -1145,6 +1135,10 @@ std::unique_ptr<Op> make_attn(const kh_launch &L, std::string &err, bool &unsupp
     // T = 1024 17.1 against 18.5 / 17.2, T = 1536 26.9 against 29.2 / 29.7 with
     // 2 / 8, T = 2048 37.8 against 43.4 / 46.1)
     else if (op->bf && groups < 16ll * current_device().cus) nw = visited <= 16 ? 2 : 4;
+    // fp16 pairs: four waves (64 KB of LDS, two workgroups per CU; GPT-2 block
+    // T = 256 6.4 us against 7.2 with 8 and 7.3 with 2, T = 1024 14.7 against
+    // 15.9 / 20.5, T = 2048 36.2 against 39.7 / 43.3)
+    if (op->f16) nw = 4;
     if (kblocks < nw) nw = kblocks >= 2 ? 2 : 1;
   }
   if (nw != 1 && nw != 2 && nw != 4 && !(nw == 8 && dh == 64)) {
@@ -1153,7 +1147,7 @@ std::unique_ptr<Op> make_attn(const kh_launch &L, std::string &err, bool &unsupp
   }
   op->nw = nw;
   // decode shapes (a few queries, a few keys): one wave per query row
-  op->rows = !op->bf && !op->in16 && tq <= kRowsMaxQ && tk <= kRowsMaxK && L.cfg[2] <= 0 && batch * tq < (1ll << 31);
+  op->rows = !op->bf && !op->in16 && !op->f16 && tq <= kRowsMaxQ && tk <= kRowsMaxK && L.cfg[2] <= 0 && batch * tq < (1ll << 31);
   const int64_t n_groups = batch * (int64_t)a.n_qblocks;
   if (n_groups >= (1ll << 31)) {
     unsupported = true;

@@ -1,0 +1,376 @@
+// kh_attn_f16.hip - the fused attention of kh_attn.hip on fp16 pairs: q, k and
+// v stored as fp16 pairs by their producer (kh_common.hpp: rows in blocks of 8
+// values, 16 bytes of h then 16 bytes of l, each scaled by a power of two),
+// both products as three fp16 MFMA passes (l.h + h.l + h.h) with fp32
+// accumulation, scores, softmax and output in fp32. The workgroup, transposed
+// scores, key split, merge and causal handling are attn_kernel's; what differs
+// is how operands reach the matrix cores:
+//   * a key block's 24 v_mfma_f32_32x32x16_f16 take 768 matrix cycles against
+//     the fp32 products' 4096, so the loads decide: each wave copies its K and
+//     V blocks into its own LDS (global_load_lds, whole rows, one block ahead;
+//     no other wave reads them, so the loop has no barrier);
+//   * K operands are 128-bit LDS reads; V^T operands (8 keys of one head
+//     dimension per lane) come from ds_read_b64_tr_b16, which transposes 4
+//     keys x 16 dimensions per 16 lanes, so V needs no transposed copy;
+//   * LDS chunks (16 bytes) of row r sit at c ^ swz_kv(r), free of bank
+//     conflicts for both reads;
+//   * the probabilities' pairs are scaled by 2^14, so that p >= 2^-15 of the
+//     row's largest splits into a full pair.
+// Two workgroups of four waves per CU (64 KB of LDS each), two waves per SIMD.
+// Measured (12 heads of 64, causal; fp32 products before): T = 512 12.0 -> 8.4
+// us, 777 23.4 -> 12.1, 1024 27.0 -> 14.7, 2048 73.7 -> 36.2; 8 heads x 600
+// queries and keys, no mask, 21.9 -> 9.7. Error against float64 the same or
+// smaller. At T = 2048, with the copies left out 27.6 us and with softmax and
+// LDS reads left out too 21.9: the matrix cores' own time at the clock they
+// hold, the tail of the causal grid and the launch; each block is copied by
+// every query block that reads it (16 KB for 24 MFMAs).
+#include <type_traits>
+
+#include "kh_attn_args.hpp"
+#include "kh_common.hpp"
+#include "kh_gemm_dev.hpp"
+#include "kh_internal.hpp"
+
+namespace kh {
+namespace {
+
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) f16x8_t lds_f16x8;
+
+// Chunk swizzle of K and V rows of DH * 4 bytes. A 128-bit read meets in one
+// LDS cycle rows {0-3, 12-15, 20-27} (kh_gemm_dev.hpp) at one chunk: 16 rows
+// distinct mod 16, so distinct slots. A transposing 64-bit read serves 32
+// lanes: 4 consecutive rows, 4 chunks 2 apart each; rows 64 wide differ in
+// chunk bits 0 and 3, rows 32 wide in the row's half of the banks and bit 0.
+template <int DH>
+__device__ __forceinline__ int swz_kv(int r) {
+  if constexpr (DH == 64) return (r & 1) | ((r & 2) << 2) | ((r >> 1) & 6);
+  else return (r >> 1) & 7;
+}
+
+template <int DH, int NW, bool ADD>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void attn_f16_kernel(const AttnArgs a) {
+  constexpr int NT = DH / 32;        // 32-wide tiles of the head dimension in O^T
+  constexpr int NC = DH / 16;        // 16-wide chunks of the head dimension in S^T
+  constexpr int RB = DH * 4;         // bytes of a row
+  constexpr int CHR = RB / 16;       // 16-byte chunks of a row
+  constexpr int RPI = 64 / CHR;      // rows one copy instruction covers
+  constexpr int NI = kKB / RPI;      // copies per block of K or V
+  constexpr int ND = DH == 64 ? 4 : 2;   // distinct swizzles among a block's copies
+  constexpr int BLOCK = kKB * RB;    // bytes of a K or V block
+  // (aligned so that a chunk's XOR stays inside its row)
+  __shared__ __attribute__((aligned(256))) float4 lds[NW * 2 * BLOCK / 16];
+  __shared__ float m_part[NW][kQB], l_part[NW][kQB];
+  static_assert(kQB * (DH + 4) * 4 <= 2 * BLOCK, "a wave's partial output fits its K and V blocks");
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int b = blockIdx.x % a.batch;
+  const int qb = a.n_qblocks - 1 - (int)(blockIdx.x / a.batch);
+  const int q0 = qb * kQB;
+  const int qi = q0 + col;
+
+  // scores in the base-2 domain: u = s * c + mask * log2(e), c >= 0 (a
+  // negative scale's sign goes into q)
+  constexpr float kLog2e = 1.4426950408889634f;
+  float c = (a.scale_mode == KH_ATTN_SCALE_MUL   ? a.scale * kLog2e
+             : a.scale_mode == KH_ATTN_SCALE_DIV ? kLog2e / a.scale
+                                                 : kLog2e) *
+            a.qk_inv;
+  const uint32_t flip = c < 0.0f ? 0x80008000u : 0u;
+  c = fabsf(c);
+
+  // Q operands: block 2 i + half of the lane's query row
+  f16x8_t qf[NC][2];
+  {
+    const float *qp = a.q + b * a.q_b + (int64_t)min(qi, a.tq - 1) * a.q_t + 8 * half;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        uint4 x = *reinterpret_cast<const uint4 *>(qp + 16 * i + 4 * p);
+        x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
+        qf[i][p] = __builtin_bit_cast(f16x8_t, x);
+      }
+  }
+
+  const bool causal = a.mask_mode == KH_ATTN_MASK_CAUSAL;
+  const int kend = causal ? min(a.tk, q0 + kQB) : a.tk;
+  const int nkb = (kend + kKB - 1) / kKB;
+  const int lim = causal ? min(a.tk, qi + 1) : a.tk;   // keys below `lim` are visible to this lane's query
+
+  // copies of block kb of an operand (head base, row stride) into LDS: row r
+  // of the block in RB bytes, chunk x at x ^ swz_kv(r). Rows past the last key
+  // repeat it (their scores are masked).
+  const int crow = lane / CHR, cpos = lane % CHR;
+  uint32_t koff[ND], voff[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const uint32_t chunk = (uint32_t)(cpos ^ swz_kv<DH>(RPI * i + crow)) * 16u;
+    koff[i] = (uint32_t)crow * (uint32_t)a.k_t * 4u + chunk;
+    voff[i] = (uint32_t)crow * (uint32_t)a.v_t * 4u + chunk;
+  }
+  const float *kbase = a.k + b * a.k_b, *vbase = a.v + b * a.v_b;
+  const uint32_t k_lds = (uint32_t)(uintptr_t)(lds_void_t *)lds + (uint32_t)(w * 2 * BLOCK), v_lds = k_lds + BLOCK;
+  // (copy i of a block; FULL: every row of the block is a key)
+  auto copy_one = [&](const float *block, const float *base, int64_t stride, const uint32_t (&off)[ND], int kb,
+                      uint32_t dst, int i, auto full) {
+    if constexpr (decltype(full)::value) {
+      copy_to_lds<4>(uniform_ptr(block + (int64_t)(RPI * i) * stride), off[i % ND], dst + i * 1024);
+    } else {
+      const uint32_t row = (uint32_t)min(kb * kKB + RPI * i + crow, a.tk - 1);
+      copy_to_lds<4>(uniform_ptr(base), row * (uint32_t)stride * 4u + (uint32_t)(cpos ^ swz_kv<DH>(RPI * i + crow)) * 16u,
+                     dst + i * 1024);
+    }
+  };
+  auto copy_k_one = [&](const float *block, int kb, int i, auto full) { copy_one(block, kbase, a.k_t, koff, kb, k_lds, i, full); };
+  auto copy_v_one = [&](const float *block, int kb, int i, auto full) { copy_one(block, vbase, a.v_t, voff, kb, v_lds, i, full); };
+  auto k_block = [&](int kb) { return kbase + (int64_t)(kb * kKB) * a.k_t; };
+  auto v_block = [&](int kb) { return vbase + (int64_t)(kb * kKB) * a.v_t; };
+  auto copy_k = [&](int kb) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) copy_k_one(nullptr, kb, i, std::false_type{});
+  };
+  auto copy_v = [&](int kb) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) copy_v_one(nullptr, kb, i, std::false_type{});
+  };
+  // copies issued before the last `later` ones have landed; LDS reads issued
+  // before this have returned (the fences keep the compiler's own LDS reads
+  // on their side of the wait)
+  auto landed = [](auto later) {
+    asm volatile("" ::: "memory");
+    wait_vmcnt<decltype(later)::value>();
+    asm volatile("" ::: "memory");
+  };
+  auto lds_reads_done = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((3 << 14) | (7 << 4) | 15);   // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  };
+  constexpr std::integral_constant<int, 0> kAll{};
+  constexpr std::integral_constant<int, NI> kAllButOneBlock{};
+
+  // K operand (chunk i, half p): chunk 4 i + 2 half + p of row col
+  const uint32_t k_at = k_lds + (uint32_t)col * RB + (uint32_t)((2 * half) ^ swz_kv<DH>(col)) * 16u;
+  auto read_k = [&](f16x8_t (&kf)[NC][2]) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) kf[i][p] = *(const lds_f16x8 *)(uintptr_t)(k_at ^ (uint32_t)((4 * i + p) * 16));
+  };
+  // V^T operand (16 keys i, tile t, half p): the lane's 8 keys are its score
+  // registers' 8 i .. 8 i + 7, i.e. keys 16 i + 8 j + 4 half + 0..3 for j = 0, 1:
+  // two transposing reads. For one of them, lane (a4 = lane % 16 / 4, b4 =
+  // lane % 4) of a 16-lane group addresses dimensions 4 b4 .. + 3 of the
+  // group's 16 in key row a4.
+  const int a4 = (lane & 15) >> 2, g1 = (lane >> 4) & 1;
+  const uint32_t v_at = v_lds + (uint32_t)(4 * half + a4) * RB +
+                        (uint32_t)((4 * g1 + (lane & 2)) ^ swz_kv<DH>(4 * half + a4)) * 16u + (uint32_t)(lane & 1) * 8u;
+  auto read_v = [&](f16x8_t (&vf)[2][NT][2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          s16x4 x[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            x[j] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_s16x4 *)(uintptr_t)((v_at ^ (uint32_t)((8 * t + p + 4 * j) * 16)) + (uint32_t)((16 * i + 8 * j) * RB)));
+          vf[i][t][p] = __builtin_shufflevector(__builtin_bit_cast(f16x4, x[0]), __builtin_bit_cast(f16x4, x[1]), 0, 1, 2,
+                                                3, 4, 5, 6, 7);
+        }
+  };
+
+  // S^T block: register r of lane (col, half) = score of query col with key
+  // (r / 4) * 8 + half * 4 + r % 4, the small products first; `between(i)`
+  // is issued behind MFMA i
+  auto scores = [&](const f16x8_t (&kf)[NC][2], auto between) {
+    f32x16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i][p == 0], qf[i][p == 1], s, 0, 0, 0);
+        between(p * NC + i);
+      }
+    return s;
+  };
+
+  f32x16 oacc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[t][r] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  // probabilities enter their pairs scaled by 2^14 (a product: added to the
+  // exponent's argument it would cost that argument 4 bits)
+  constexpr float kUp = 16384.0f;
+
+  // Online softmax of one block, in place (see attn_kernel); only a wave's
+  // last block can hold keys past the causal diagonal or the last key.
+  auto softmax = [&](f32x16 &s, int kb, auto masked) {
+    constexpr bool kU = ADD || decltype(masked)::value;   // s holds u, not the raw scores
+    const int room = lim - kb * kKB - half * 4;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float u = s[r];
+      if constexpr (ADD) {
+        const int key = min(kb * kKB + half * 4 + (r >> 2) * 8 + (r & 3), a.tk - 1);
+        u = fmaf(u, c, a.mask[b * a.m_b + (int64_t)min(qi, a.tq - 1) * a.m_q + (int64_t)key * a.m_k] * kLog2e);
+      } else if constexpr (kU) {
+        u *= c;
+      }
+      if constexpr (decltype(masked)::value) u = (r >> 2) * 8 + (r & 3) < room ? u : -INFINITY;
+      s[r] = u;
+      mx = fmaxf(mx, u);
+    }
+    const float2 mh = halves(mx);
+    mx = fmaxf(mh.x, mh.y);
+    const float m_new = fmaxf(m_run, kU ? mx : mx * c);
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f(kU ? s[r] - m_use : fmaf(s[r], c, -m_use));
+      part[r & 3] += s[r];
+    }
+    const float2 sh = halves((part[0] + part[1]) + (part[2] + part[3]));
+    l_run = fmaf(l_run, alpha, sh.x + sh.y);
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) oacc[t] *= alpha;
+  };
+  // O^T += V^T P^T: a lane's P operand is its own score registers
+  auto pv = [&](const f16x8_t (&vf)[2][NT][2], const f32x16 &p) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint4 h, l;
+      split_f16x2(p[8 * i] * kUp, p[8 * i + 1] * kUp, h.x, l.x);
+      split_f16x2(p[8 * i + 2] * kUp, p[8 * i + 3] * kUp, h.y, l.y);
+      split_f16x2(p[8 * i + 4] * kUp, p[8 * i + 5] * kUp, h.z, l.z);
+      split_f16x2(p[8 * i + 6] * kUp, p[8 * i + 7] * kUp, h.w, l.w);
+      const f16x8_t ph = __builtin_bit_cast(f16x8_t, h), pl = __builtin_bit_cast(f16x8_t, l);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][1], ph, oacc[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][0], pl, oacc[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][0], ph, oacc[t], 0, 0, 0);
+    }
+  };
+
+  // This wave's key blocks w, w + NW, ...: the next block's scores are issued
+  // ahead of the current one's softmax, so the matrix cores work through the
+  // exponentials. Copies run a block ahead; the last ones repeat a block that
+  // is not read (so the counts stay fixed) and are waited for at the end.
+  int kb = w;
+  if (kb < nkb) {
+    f16x8_t kf[NC][2], vf[2][NT][2];
+    copy_k(kb);
+    copy_v(kb);
+    landed(kAllButOneBlock);
+    read_k(kf);
+    lds_reads_done();
+    copy_k(min(kb + NW, nkb - 1));
+    f32x16 s_cur = scores(kf, [](int) {});
+    auto loop = [&](auto full) {
+      for (; kb + NW < nkb; kb += NW) {
+        landed(kAll);   // K of the next block and V of this one, copied a block ago
+        read_k(kf);
+        read_v(vf);
+        lds_reads_done();
+        const int k2 = min(kb + 2 * NW, nkb - 1), v1 = kb + NW;
+        const float *kp = k_block(k2), *vp = v_block(v1);
+        // the copies are spread over the score MFMAs
+        const f32x16 s_nxt = scores(kf, [&](int i) {
+#pragma unroll
+          for (int x = 0; x < 2 * NI; ++x) {
+            if (x * 3 * NC / (2 * NI) != i) continue;
+            if (x < NI) copy_k_one(kp, k2, x, full);
+            else copy_v_one(vp, v1, x - NI, full);
+          }
+        });
+        softmax(s_cur, kb, std::false_type{});
+        pv(vf, s_cur);
+        s_cur = s_nxt;
+      }
+    };
+    if (nkb * kKB <= a.tk) loop(std::true_type{});
+    else loop(std::false_type{});
+    landed(kAll);
+    read_v(vf);
+    softmax(s_cur, kb, std::true_type{});
+    pv(vf, s_cur);
+    lds_reads_done();
+  }
+
+  // merge the NW key-split partials (each wave's in its own blocks of LDS):
+  // o = sum_w 2^(m_w - M) o_w / sum_w 2^(m_w - M) l_w
+  float *mine = reinterpret_cast<float *>(lds) + w * (2 * BLOCK / 4);
+  if (half == 0) m_part[w][col] = m_run, l_part[w][col] = l_run;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<float4 *>(mine + col * (DH + 4) + t * 32 + 2 * r + half * 4) =
+          make_float4(oacc[t][r], oacc[t][r + 1], oacc[t][r + 2], oacc[t][r + 3]);
+  __syncthreads();
+  constexpr int kChunks = kQB * DH / 4;
+  for (int x = threadIdx.x; x < kChunks; x += 64 * NW) {
+    const int qr = x / (DH / 4), d = (x % (DH / 4)) * 4;
+    if (q0 + qr >= a.tq) continue;
+    float mm = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) mm = fmaxf(mm, m_part[u][qr]);
+    const float mu = mm == -INFINITY ? 0.0f : mm;
+    float l = 0.0f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      const float e = __builtin_amdgcn_exp2f(m_part[u][qr] - mu);
+      const float4 o = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(lds) + u * (2 * BLOCK / 4) +
+                                                         qr * (DH + 4) + d);
+      l += l_part[u][qr] * e;
+      acc.x += o.x * e, acc.y += o.y * e, acc.z += o.z * e, acc.w += o.w * e;
+    }
+    const float back = a.v_inv / kUp;
+    const float4 out = make_float4(acc.x / l * back, acc.y / l * back, acc.z / l * back, acc.w / l * back);
+    float *row = a.o + b * a.o_b + (int64_t)(q0 + qr) * a.o_t;
+    if (a.o_pair) store_f16_pairs4(row, d, out, a.o_scale);
+    else *reinterpret_cast<float4 *>(row + d) = out;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_attn_f16(const AttnArgs &a, int dh, int nw, dim3 grid, hipStream_t stream) {
+#define KH_ATTN_F16_LAUNCH(D, W)                                                                     \
+  if (dh == D && nw == W) {                                                                          \
+    if (a.mask_mode == KH_ATTN_MASK_ADD)                                                             \
+      hipLaunchKernelGGL((attn_f16_kernel<D, W, true>), grid, dim3(64 * W), 0, stream, a);          \
+    else                                                                                             \
+      hipLaunchKernelGGL((attn_f16_kernel<D, W, false>), grid, dim3(64 * W), 0, stream, a);         \
+    return hipGetLastError();                                                                        \
+  }
+  KH_ATTN_F16_LAUNCH(64, 8)
+  KH_ATTN_F16_LAUNCH(64, 4)
+  KH_ATTN_F16_LAUNCH(64, 2)
+  KH_ATTN_F16_LAUNCH(64, 1)
+  KH_ATTN_F16_LAUNCH(32, 4)
+  KH_ATTN_F16_LAUNCH(32, 2)
+  KH_ATTN_F16_LAUNCH(32, 1)
+#undef KH_ATTN_F16_LAUNCH
+  return hipErrorInvalidValue;
+}
+
+}  // namespace kh

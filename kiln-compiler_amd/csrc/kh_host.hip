@@ -218,7 +218,8 @@ void attend(int64_t tk, int64_t dh, int scale_mode, float scale, int mask_mode, 
   // three-pass sum lo.hi + hi.lo + hi.hi of the bf16 halves (a non-finite hi
   // keeps lo 0)
   auto prod = [prec](float x, float y) -> double {
-    if (prec == 0) return (double)x * (double)y;
+    // (fp16 pairs hold 23 bits of each input: taken as exact here)
+    if (prec == 0 || prec == 3) return (double)x * (double)y;
     const float xh = bf16_round(x), yh = bf16_round(y);
     if (prec == 1) return (double)xh * (double)yh;
     const float xl = std::isfinite(xh) ? bf16_round(x - xh) : 0.0f, yl = std::isfinite(yh) ? bf16_round(y - yh) : 0.0f;
@@ -245,8 +246,8 @@ void attend(int64_t tk, int64_t dh, int scale_mode, float scale, int mask_mode, 
   for (int64_t d = 0; d < dh; ++d) {
     double acc = 0.0;
     for (int64_t j = 0; j < tk; ++j)
-      acc += prec ? prod((float)(s[j] / l), v[j * v_sj + d * v_sd]) : s[j] * (double)v[j * v_sj + d * v_sd];
-    out[d] = prec ? acc : acc / l;
+      acc += prec == 1 || prec == 2 ? prod((float)(s[j] / l), v[j * v_sj + d * v_sd]) : s[j] * (double)v[j * v_sj + d * v_sd];
+    out[d] = prec == 1 || prec == 2 ? acc : acc / l;
   }
 }
 

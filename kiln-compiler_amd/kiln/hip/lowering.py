@@ -57,6 +57,11 @@ ATTN_ROWS_MAX_Q = 4
 # 16-query kernel, which is faster there (T = 256 6.8 against 7.9 us, T = 128
 # 5.2 against 5.8)
 ATTN_X3_MIN_GROUPS = 192
+# fp32 plans run attention on fp16 pairs from this many keys on (GPT-2 block,
+# 12 heads causal: T = 256 6.9 -> 6.4 us, 512 12.0 -> 8.4, 1024 27.0 -> 14.7,
+# 2048 73.7 -> 36.2); below, the 16-query fp32 kernel spreads over more
+# workgroups (T = 128 4.9 against 5.2 us)
+ATTN_F16_MIN_KEYS = 160
 
 _UNARY_OP = {"neg": "neg", "exp": "exp", "tanh": "tanh", "sigmoid": "sigmoid", "relu": "relu",
              "rsqrt": "rsqrt", "sqrt": "sqrt", "erf": "erf", "copy": "mov"}
@@ -403,6 +408,36 @@ class _Lowerer:
             if k.kind == "matmul" and k not in self.prologue and self.matmul_choice(k)[1] == "f16x3":
                 buf, e = self.f16_operand(k)
                 out[buf] = e
+            elif k.kind == "attention":
+                out.update(self.f16_attention(k) or {})
+        return out
+
+    def f16_attention(self, k):
+        """{arena buffer: exponent of its scale} of attention kernel k's q, k and
+        v if it can run on fp16 pairs: each a view with unit head-dim stride
+        and rows of whole 32-byte blocks of a bounded buffer that k alone reads
+        and a matrix product writes as pairs; enough keys. Else None."""
+        from kiln.hip.attention import match_kernel, operand_strides
+
+        m = match_kernel(self.g, k)
+        strides = operand_strides(m, self.layouts) if m is not None else None
+        if (strides is None or m.q.shape[1] <= ATTN_ROWS_MAX_Q or ATTN_QUERIES == 16
+                or m.v.shape[1] < ATTN_F16_MIN_KEYS):
+            return None
+        out = {}
+        for v, (offset, st) in zip((m.q, m.k, m.v), strides):
+            lay = self.layouts.get(v)
+            if lay is None or lay.base[0] != "arena" or offset % 8 or st[0] % 8 or st[1] % 8:
+                return None
+            buf = lay.base[1]
+            producer = self.g.kernel_of(buf.node)
+            if (self._arena_readers().get(buf) != {k} or buf in self.g.results or producer is None
+                    or producer.kind != "matmul"):
+                return None
+            e = f16.activation_exponent(self.bounds.largest(buf))
+            if e is None or not self._writes_f16(producer, buf):
+                return None
+            out[buf] = e
         return out
 
     def f16_operand(self, k):
@@ -1617,9 +1652,10 @@ class _Lowerer:
                 d.cfg[7] |= 1 << j
             if self.stored_pairs(v):  # (pair words: addressed as fp32)
                 d.cfg[7] |= 1 << (16 + j)
-            if self.stored_f16(v) is not None:   # the output
+            if self.stored_f16(v) is not None:   # q, k and v together, the output
                 d.cfg[7] |= 1 << (16 + j)
-                d.cfg[6], d.fparams[3] = kl.PAIR_F16, 2.0 ** self.stored_f16(v)
+                if j == 3:
+                    d.cfg[6], d.fparams[3] = kl.PAIR_F16, 2.0 ** self.stored_f16(v)
             d.refs[j] = r
         d.n_refs = 4
         mode = kl.ATTN_MASK_NONE
@@ -1641,6 +1677,11 @@ class _Lowerer:
             d.cfg[5] = 1
         if x3_products:
             d.cfg[5] = 2
+        f16_products = self.stored_f16(m.q) is not None
+        if f16_products:
+            d.cfg[5] = 3
+            d.fparams[1] = 2.0 ** -(self.stored_f16(m.q) + self.stored_f16(m.k))
+            d.fparams[2] = 2.0 ** -self.stored_f16(m.v)
         d.fparams[0] = m.scale
         causal = mode == kl.ATTN_MASK_CAUSAL
         pairs = sum(min(tk, i + 1) for i in range(tq)) if causal else tq * tk
@@ -1659,7 +1700,9 @@ class _Lowerer:
         if d.cfg[7] & 8:
             scale += ", out:bf16"
             nbytes -= 2 * batch * dh * tq
-        if d.cfg[7] >> 16 & 7:
+        if f16_products:
+            scale += ", products:f16x3"
+        elif d.cfg[7] >> 16 & 7:
             scale += ", qkv:pairs"
         if d.cfg[7] >> 16 & 8:
             scale += ", out:f16" if d.cfg[6] == kl.PAIR_F16 else ", out:pairs"

@@ -104,6 +104,64 @@ def test_rows_of_any_size_and_non_finite_rows(loc, scale):
     np.testing.assert_allclose(out[good].cpu().numpy(), plain[good].cpu().numpy(), rtol=RTOL, atol=ATOL)
 
 
+class _Attention(torch.nn.Module):
+    """LayerNorm -> q, k, v (one product) -> attention, heads merged."""
+
+    def __init__(self, d, heads, tokens, mask, scale):
+        super().__init__()
+        self.heads, self.scale = heads, scale
+        self.ln, self.qkv = torch.nn.LayerNorm(d), torch.nn.Linear(d, 3 * d)
+        with torch.no_grad():
+            self.qkv.weight.normal_(0.0, 1.0 / d ** 0.5), self.qkv.bias.normal_(0.0, 0.1)
+        if mask == "causal":
+            self.register_buffer("mask", torch.full((tokens, tokens), float("-inf")).triu(1))
+        elif mask == "add":
+            m = torch.randn(tokens, tokens).masked_fill(torch.rand(tokens, tokens) < 0.3, float("-inf"))
+            m[5] = float("-inf")     # a row that sees no key: NaN, as in eager
+            self.register_buffer("mask", m)
+        else:
+            self.mask = None
+
+    def forward(self, x):
+        t, c = x.shape
+        q, k, v = (y.view(t, self.heads, c // self.heads).transpose(0, 1) for y in self.qkv(self.ln(x)).split(c, dim=1))
+        s = (q @ k.transpose(-2, -1)) * self.scale
+        s = s if self.mask is None else s + self.mask
+        return (F.softmax(s, dim=-1) @ v).transpose(0, 1).contiguous().view(t, c)
+
+
+# keys from the fewest that take the path: whole blocks, one past, one short;
+# both head dims; a negative and a zero scale; fully masked rows
+@pytest.mark.parametrize("tokens,d,heads,mask,scale", [
+    (160, 128, 2, None, 0.125), (161, 128, 4, "causal", 0.17), (191, 64, 2, "causal", 0.17), (192, 64, 1, "add", 0.125),
+    (333, 256, 4, "causal", 0.125), (333, 256, 8, "add", 0.17), (257, 128, 2, None, -0.2), (200, 128, 2, "causal", 0.0),
+    (1025, 128, 2, "causal", 0.125)])
+def test_attention_on_pairs(tokens, d, heads, mask, scale, monkeypatch):
+    from kiln.hip import lowering
+
+    torch.manual_seed(tokens)
+    model, x = _Attention(d, heads, tokens, mask, scale).eval(), torch.randn(tokens, d)
+
+    def run():
+        c = kiln.compile(model, (x,), device="cuda", cuda_graphs=False, plan_cache=False)
+        return c, c(x.cuda())
+
+    c, out = run()
+    assert any("products:f16x3" in l.summary for l in c._exe.program.launches)
+    monkeypatch.setattr(lowering._Lowerer, "f16_attention", lambda self, k: None)
+    _, plain = run()
+    with torch.no_grad():
+        ref = model.double()(x.double())
+    out, plain = out.cpu().double(), plain.cpu().double()
+    bad = torch.isnan(ref)
+    assert torch.equal(torch.isnan(out), bad)
+    np.testing.assert_allclose(out[~bad].numpy(), ref[~bad].numpy(), rtol=RTOL, atol=ATOL)
+    err, err_plain = ((t - ref)[~bad].norm() / ref[~bad].norm() for t in (out, plain))
+    assert err <= 1.1 * err_plain, (err, err_plain)
+    for _ in range(3):
+        assert torch.equal(c(x.cuda()).cpu().double()[~bad], out[~bad])
+
+
 @pytest.mark.parametrize("T", [16, 300, 777])
 def test_block_on_pairs(T):
     model = gpt2_init_(Block(256, 4, T), seed=0).eval()
