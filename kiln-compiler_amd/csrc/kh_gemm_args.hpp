@@ -182,7 +182,7 @@ inline hipError_t launch_splitk_reduce(const GemmArgs &a, int cus, hipStream_t s
 // per workgroup): id, BM x BN, waves WM x WN, stages NS.
 #define KH_GEMM_F16_CONFIGS(X) \
   X(101, 128, 192, 2, 4, 3)    \
-  X(102, 64, 96, 2, 2, 3)      \
+  X(102, 64, 96, 2, 2, 4)      \
   X(103, 64, 64, 2, 2, 2)      \
   X(104, 32, 96, 2, 2, 4)      \
   X(105, 32, 64, 2, 2, 4)
@@ -227,10 +227,11 @@ constexpr int kLnMaxK = 1024;
 
 // The same kernel over fp16 pairs (precision 3).
 #define KH_GEMM_SMALL_F16_CONFIGS(X) \
-  X(106, 16, 32, 8, 2, 3)            \
+  X(106, 16, 32, 8, 3, 3)            \
   X(107, 32, 32, 4, 2, 3)            \
-  X(108, 32, 48, 4, 2, 3)            \
-  X(109, 16, 16, 4, 2, 3)
+  X(108, 32, 48, 4, 3, 3)            \
+  X(109, 16, 32, 4, 3, 3)            \
+  X(110, 16, 16, 8, 4, 3)
 
 // Launch configuration `id` of kind 6 (hipErrorInvalidValue for another id).
 hipError_t launch_gemm_small(int id, const GemmArgs &a, dim3 grid, hipStream_t stream);

@@ -163,7 +163,7 @@ TILES = {
     99: (64, 64, 64, 2, 2, 1, 16),
     100: (128, 96, 64, 2, 2, 1, 16),
     # fp32 products on fp16 pairs: one tile per workgroup (101-105), and the
-    # small-M kernel (106-109)
+    # small-M kernel (106-110)
     101: (128, 192, 32, 2, 4, 1, 16),
     102: (64, 96, 32, 2, 2, 1, 16),
     103: (64, 64, 32, 2, 2, 1, 16),
@@ -172,7 +172,8 @@ TILES = {
     106: (16, 32, 32, 1, 1, 8, 16),
     107: (32, 32, 32, 1, 1, 4, 16),
     108: (32, 48, 32, 1, 1, 4, 16),
-    109: (16, 16, 32, 1, 1, 4, 16),
+    109: (16, 32, 32, 1, 1, 4, 16),
+    110: (16, 16, 32, 1, 1, 8, 16),
 }
 # configurations of the skinny-M kernel: A row-major with unit K stride and
 # K % 4 == 0, B a constant read through its [batch][N][K] copy, no split-K;
@@ -189,7 +190,7 @@ BF16_A = frozenset(range(95, 101))
 # configurations of the small-M kernel: as the K-contiguous pipeline (B the
 # [batch][N][K] copy, K a positive multiple of 32, no split-K), for products
 # with at most SMALL_M_MAX rows
-SMALL_M = frozenset(range(65, 87)) | frozenset(range(106, 110))
+SMALL_M = frozenset(range(65, 87)) | frozenset(range(106, 111))
 SMALL_M_MAX = 1024
 # configurations that read B through its [batch][N][K] copy
 NK_B = SKINNY | K_CONTIGUOUS | SMALL_M
@@ -219,7 +220,7 @@ OCCUPANCY = {0: 2, 1: 2, 2: 3, 3: 2, 4: 4, 5: 2, 6: 1, 7: 1, 8: 4, 9: 4, 10: 4, 
              75: 4, 76: 2, 77: 3, 78: 3, 79: 4, 80: 3, 81: 2, 82: 2, 83: 4, 84: 2, 85: 1, 86: 2,
              87: 1, 88: 1, 89: 1, 90: 1, 91: 1, 92: 1, 93: 1, 94: 1,
              95: 1, 96: 1, 97: 1, 98: 1, 99: 1, 100: 1,
-             101: 1, 102: 2, 103: 3, 104: 2, 105: 3, 106: 1, 107: 2, 108: 2, 109: 4}
+             101: 1, 102: 2, 103: 3, 104: 2, 105: 3, 106: 1, 107: 2, 108: 1, 109: 2, 110: 1}
 EFFICIENCY = {0: 0.62, 1: 0.6, 2: 0.62, 3: 0.58, 4: 0.66, 5: 0.62, 6: 0.67, 7: 0.55,
               8: 0.55, 9: 0.55, 10: 0.5, 11: 0.5, 12: 0.45, 13: 0.5, 14: 0.55,
               15: 0.15, 16: 0.15, 17: 0.15, 18: 0.15, 19: 0.15, 20: 0.15,
@@ -234,14 +235,19 @@ EFFICIENCY = {0: 0.62, 1: 0.6, 2: 0.62, 3: 0.58, 4: 0.66, 5: 0.62, 6: 0.67, 7: 0
               84: 0.1, 85: 0.12, 86: 0.2,
               87: 0.2, 88: 0.2, 89: 0.2, 90: 0.2, 91: 0.2, 92: 0.35, 93: 0.35, 94: 0.35,
               95: 0.3, 96: 0.28, 97: 0.26, 98: 0.26, 99: 0.25, 100: 0.26,
-              **{t: 0.35 for t in range(101, 110)}}
-# Measured times of the fp16-pair configurations (GPT-2 shapes, M 128 to 2048,
-# K 768 and 3072): microseconds a launch takes beyond its K steps (launch,
-# first loads, output), and microseconds per 32-deep step for every tile that
-# falls to a CU (the matrix cores, the copies into LDS and the tiles sharing
-# the CU go at that rate whatever their number)
-F16_TIMES = {101: (9.5, 0.97), 102: (6.0, 0.31), 103: (5.5, 0.20), 104: (5.5, 0.17), 105: (4.5, 0.13),
-             106: (3.4, 0.047), 107: (3.2, 0.086), 108: (4.6, 0.125), 109: (3.3, 0.031)}
+              **{t: 0.35 for t in range(101, 111)}}
+# Times of the fp16-pair configurations, fitted to whole GPT-2 blocks and MLPs
+# (27 to 2048 rows, widths 256 to 1024) timed with each tile in each product's
+# place, so that A is what the launch before has just written: microseconds
+# of a launch beyond its K steps; per 32-deep step, for every tile that falls
+# to a CU and at least for every round of workgroups; and per further round.
+# The model's pick costs 0.3 us more than the best tile on average over the
+# 58 products it was fitted to (64 x 96 tiles of 4096 columns, 5 to 8 us more
+# than 64 x 64, are its worst).
+F16_TIMES = {101: (9.7, 0.550, 0.602, 4.0), 102: (6.8, 0.190, 0.201, 5.9), 103: (4.2, 0.159, 0.400, 3.4),
+             104: (4.5, 0.153, 0.167, 2.3), 105: (4.1, 0.115, 0.137, 0.7), 106: (3.5, 0.044, 0.062, 1.2),
+             107: (3.5, 0.071, 0.131, 1.7), 108: (5.2, 0.087, 0.110, 3.1), 109: (3.8, 0.062, 0.070, 0.5),
+             110: (3.7, 0.024, 0.041, 1.4)}
 # the one whose products sum in a single chain (the others keep the small
 # products apart): for as many rows as the fp32 kernels summed so themselves
 F16_SINGLE_CHAIN = 101
@@ -302,10 +308,11 @@ def estimate(tile, splitk, batch, m, n, k, cus) -> float:  # noqa: C901
     CU's matrix cores), plus the split-K reduce (partials through HBM)."""
     bm, bn, bk = TILES[tile][:3]
     if tile in F16_TIMES:
-        launch, step = F16_TIMES[tile]
+        launch, step, latency, more = F16_TIMES[tile]
         tiles = math.ceil(m / bm) * math.ceil(n / bn) * batch
         rounds = math.ceil(tiles / (cus * OCCUPANCY[tile]))
-        return launch * rounds + math.ceil(tiles / cus) * math.ceil(k / bk) * step
+        per_step = max(math.ceil(tiles / cus) * step, rounds * latency)
+        return launch + more * (rounds - 1) + math.ceil(k / bk) * per_step
     units = math.ceil(m / bm) * math.ceil(n / bn) * batch * splitk
     rounds = math.ceil(units / (cus * OCCUPANCY[tile]))
     kper = math.ceil(k / splitk / bk) * bk
@@ -438,16 +445,18 @@ LN_EPS = 1e-5
 class _Trial:
     """One candidate configuration, built and checked, ready to be timed."""
 
-    def __init__(self, config, exe, inputs, output):
+    def __init__(self, config, exe, inputs, output, chain=False):
         self.config = config
         self.exe = exe
         self.ins = [t.data_ptr() for t in inputs]
         self.outs = [output.data_ptr()]
         self.best = float("inf")
-        # the product's own launches (a LayerNorm in front of it is not timed)
+        # the product's own launches (a LayerNorm in front of it is not timed;
+        # with `chain` it is, so the product reads what was just written: in a
+        # block its A is in no XCD's L2, which decides the ring's depth)
         names = [launch.name for launch in exe.program.launches]
         mm = [i for i, name in enumerate(names) if "matmul" in name]
-        self.index = mm[0] if len(names) > 1 and len(mm) == 1 else -1
+        self.index = mm[0] if len(names) > 1 and len(mm) == 1 and not chain else -1
 
     @property
     def key(self):
@@ -566,7 +575,7 @@ class GPUAutotuner:
                 rejected.append(f"{config}: {type(failure).__name__}: {first}")
                 continue
             if err <= tolerance:
-                trials.append(_Trial(config, exe, [x_dev], out))
+                trials.append(_Trial(config, exe, [x_dev], out, chain=precision == "f16x3"))
             else:
                 rejected.append(f"{config}: relative error {err:.1e}")
         return trials, rejected
