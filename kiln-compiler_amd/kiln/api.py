@@ -259,6 +259,8 @@ class CompiledModule:
     def _graph_args(self, inputs):
         if len(inputs) != len(self._free):
             raise TypeError(f"expected {len(self._free)} inputs, got {len(inputs)}")
+        if not self._bound:   # every graph argument is a runtime input
+            return inputs
         args = [None] * len(self.graph.args)
         for slot, t in zip(self._free, inputs):
             args[slot] = t

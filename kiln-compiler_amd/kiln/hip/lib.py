@@ -178,11 +178,15 @@ def device_info():
     return {"cus": cus.value, "lds_bytes": lds.value, "arch": arch.value.decode()}
 
 
+_pointer_types = {}   # number of pointers -> ctypes array type (making one costs more than an array of it)
+
+
 def pointer_array(ptrs):
-    arr = (ctypes.c_void_p * max(1, len(ptrs)))()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    n = len(ptrs)
+    kind = _pointer_types.get(n)
+    if kind is None:
+        kind = _pointer_types[n] = ctypes.c_void_p * max(1, n)
+    return kind(*ptrs)
 
 
 class Plan:
@@ -208,8 +212,10 @@ class Plan:
               "kh_plan_bind")
 
     def run(self, in_ptrs, out_ptrs, stream):
-        ins, outs = pointer_array(in_ptrs), pointer_array(out_ptrs)
-        check(self.lib.kh_plan_run(self.handle, ins, len(in_ptrs), outs, len(out_ptrs), stream), "kh_plan_run")
+        rc = self.lib.kh_plan_run(self.handle, pointer_array(in_ptrs), len(in_ptrs), pointer_array(out_ptrs),
+                                  len(out_ptrs), stream)
+        if rc:
+            check(rc, "kh_plan_run")
 
     def run_host(self, in_ptrs, out_ptrs):
         """The plan executed on the CPU over host buffers (kh_plan_run_host)."""

@@ -60,7 +60,9 @@ def check_memory(dev, needed_bytes, what):
 
 
 def current_stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream (without building a Stream object
+    around it, which costs about as much as a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class _ReplayTimer:
@@ -209,7 +211,7 @@ class HIPExecutable:
             raise TypeError(f"expected {len(self.input_shapes)} inputs, got {len(inputs)}")
         ready = []
         for i, (t, shape) in enumerate(zip(inputs, self.input_shapes)):
-            if tuple(t.shape) != shape:
+            if t.shape != shape:   # (a torch.Size compares as the tuple it is)
                 raise ValueError(f"Kiln was compiled for input shape {shape}, got {tuple(t.shape)} (input {i})")
             if t.device != self.device or t.dtype != torch.float32 or not t.is_contiguous():
                 t = t.detach().to(device=self.device, dtype=torch.float32).contiguous()
@@ -298,7 +300,7 @@ class HIPExecutable:
 
     def __call__(self, *inputs):
         inputs = self._prepare(inputs)
-        capturing = torch.cuda.is_current_stream_capturing()
+        capturing = torch._C._cuda_isCurrentStreamCapturing()
         if not self.use_cuda_graphs or capturing or self.debug:
             out = self._direct(inputs)   # also inside a caller's own stream capture; debug runs launch by launch
         else:
