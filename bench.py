@@ -222,7 +222,9 @@ def dominant_kernel_roofline(compiled, x, T):
     avg_ms = min(events_ms(fn, 200) for _ in range(3))
     if launch.flops:
         achieved = launch.flops / (avg_ms * 1e-3) / 1e12
-        bound, peak, unit = "mfma", FP32_PEAK_TFLOPS, "TFLOP/s"
+        # an fp32 product on fp16 pairs is three fp16 MFMA passes
+        on_pairs = "f16x3" in launch.summary
+        bound, peak, unit = "mfma", round(BF16_PEAK_TFLOPS / 3, 1) if on_pairs else FP32_PEAK_TFLOPS, "TFLOP/s"
     else:
         achieved = launch.bytes / (avg_ms * 1e-3) / 1e9
         bound, peak, unit = "hbm", HBM_PEAK_GBS, "GB/s"

@@ -38,41 +38,49 @@ def padded_k(k: int) -> int:
     return (k + 7) // 8 * 8
 
 
-def _rows(data: np.ndarray, offset: int, strides, batch: int, k: int, n: int) -> torch.Tensor:
+def _rows(data: np.ndarray, offset: int, strides, batch: int, k: int, n: int, device) -> torch.Tensor:
     """The [batch, K, N] view (element offset, strides over (b, k, n)) of a
-    constant as float32 [batch, N, K] (a view)."""
-    flat = torch.from_numpy(np.ascontiguousarray(data, dtype=np.float32).reshape(-1))
+    constant as float32 [batch, N, K] on `device` (a view)."""
+    flat = torch.from_numpy(np.ascontiguousarray(data, dtype=np.float32).reshape(-1)).to(device)
     sb, sk, sn = (int(s) for s in strides)
     return torch.as_strided(flat, (batch, n, k), (sb, sn, sk), offset)
 
 
-def row_exponents(data, offset, strides, batch: int, k: int, n: int) -> torch.Tensor:
-    """e [batch, N] (int32): a row's largest magnitude times 2^e lands in
-    [2^TOP, 2^(TOP + 1))."""
-    rows = _rows(data, offset, strides, batch, k, n)
-    top = torch.maximum(rows.amax(dim=-1), -rows.amin(dim=-1)) if k else torch.zeros(batch, n)
+def row_exponents(rows: torch.Tensor) -> torch.Tensor:
+    """e [batch, N] (int32) of float32 [batch, N, K]: a row's largest magnitude
+    times 2^e lands in [2^TOP, 2^(TOP + 1))."""
+    top = torch.maximum(rows.amax(dim=-1), -rows.amin(dim=-1))
     _, exponent = torch.frexp(top)   # top in [2^(exponent - 1), 2^exponent)
     return torch.where(top > 0, TOP + 1 - exponent, torch.zeros_like(exponent)).clamp(*WEIGHT_EXPONENTS)
 
 
-def pair_rows(data, offset, strides, batch: int, k: int, n: int) -> np.ndarray:
-    """The [batch, N, K'] pair copy (int32 words) of the [batch, K, N] view of
-    a constant, each row times its own power of two (row_exponents)."""
-    e = row_exponents(data, offset, strides, batch, k, n)
-    rows = _rows(data, offset, strides, batch, k, n).contiguous()
-    rows = rows * torch.ldexp(torch.ones(()), e).unsqueeze(-1)
+def _power_of_two(e: torch.Tensor) -> torch.Tensor:
+    """float32 2^e, |e| <= 126, from its bits (torch.ldexp goes through pow,
+    which the GPU does not round to an exact power)."""
+    return ((e.int() + 127) << 23).view(torch.float32)
+
+
+def pair_rows(data, offset, strides, batch: int, k: int, n: int, device="cpu") -> torch.Tensor:
+    """The [batch, N, K'] pair copy (int32 words, on `device`) of the [batch, K,
+    N] view of a constant, each row times its own power of two (row_exponents).
+    The same bits on the CPU and on the GPU, where it is ~100 times faster."""
+    rows = _rows(data, offset, strides, batch, k, n, device)
+    rows = rows.contiguous() * _power_of_two(row_exponents(rows)).unsqueeze(-1)
     kp = padded_k(k)
     if kp != k:
         rows = torch.nn.functional.pad(rows, (0, kp - k))
     rows = rows.view(batch, n, kp // 8, 8)
-    blocks = torch.empty(batch, n, kp // 8, 2, 8, dtype=torch.float16)
-    blocks[:, :, :, 0] = rows   # (rounds to nearest)
-    blocks[:, :, :, 1] = rows.sub_(blocks[:, :, :, 0])
-    return blocks.numpy().view(np.int32).reshape(batch, n, kp)
+    h = rows.half()   # (rounds to nearest)
+    l = (rows - h.float()).half()
+    return torch.stack([h, l], dim=3).view(torch.int32).view(batch, n, kp)
 
 
-def column_scales(data, offset, strides, batch: int, k: int, n: int, activation_e: int) -> np.ndarray:
+def column_scales(data, offset, strides, batch: int, k: int, n: int, activation_e: int, device="cpu") -> torch.Tensor:
     """2^-(e + activation_e) per column (float32 [batch, N]): what a product of
     the scaled operands is multiplied by."""
-    e = row_exponents(data, offset, strides, batch, k, n).numpy()
-    return np.ldexp(np.float32(1.0), -(e + activation_e)).astype(np.float32)
+    e = row_exponents(_rows(data, offset, strides, batch, k, n, device))
+    return _power_of_two(-(e + activation_e))
+
+
+def pair_bytes(batch: int, k: int, n: int) -> int:
+    return 4 * batch * n * padded_k(k)

@@ -113,6 +113,17 @@ def nk_copy(data: np.ndarray, offset: int, strides, batch: int, k: int, n: int) 
     return np.ascontiguousarray(view)
 
 
+def _on_pairs(name: str) -> bool:
+    return "@f16:" in name or "@f16s:" in name
+
+
+def pair_constant(recipe, constants: dict, name: str, where) -> torch.Tensor:
+    """The fp16-pair copy of a weight, or its columns' scales, made on `where`."""
+    src, offset, strides, batch, k, n = recipe[:6]
+    args = (constants[src], offset, strides, batch, k, n)
+    return f16.pair_rows(*args, where) if "@f16:" in name else f16.column_scales(*args, recipe[6][1], where)
+
+
 def host_constant(program, constants: dict, name: str) -> np.ndarray:
     """Host array for const slot ``name``: the fp32 constant itself, or the
     copy the lowering asked to derive from one (``program.derived``)."""
@@ -120,9 +131,8 @@ def host_constant(program, constants: dict, name: str) -> np.ndarray:
     if recipe is None:
         return np.ascontiguousarray(constants[name], np.float32)
     src, offset, strides, batch, k, n = recipe[:6]
-    if "@f16:" in name or "@f16s:" in name:
-        args = (constants[src], offset, strides, batch, k, n)
-        return f16.pair_rows(*args) if "@f16:" in name else f16.column_scales(*args, recipe[6][1])
+    if _on_pairs(name):
+        return pair_constant(recipe, constants, name, "cpu").numpy()
     if "@nk:" in name:
         return nk_copy(constants[src], offset, strides, batch, k, n)
     if "@nkg:" in name or "@lnc:" in name or "@lng:" in name:
@@ -160,8 +170,13 @@ class HIPExecutable:
         self.debug = debug
 
         self.plan = kl.Plan([launch.desc for launch in program.launches])
-        host = [host_constant(program, constants, name) for name in program.consts]
-        self.weight_bytes = sum(int(h.nbytes) for h in host)
+        # (fp16-pair copies are made on the device, below)
+        host = [None if _on_pairs(name) else host_constant(program, constants, name) for name in program.consts]
+        self.weight_bytes = sum(int(h.nbytes) for h in host if h is not None)
+        for name in program.consts:
+            if _on_pairs(name):
+                batch, k, n = program.derived[name][3:6]
+                self.weight_bytes += f16.pair_bytes(batch, k, n) if "@f16:" in name else 4 * batch * n
         self.arena_bytes = arena_bytes
         ws = self.plan.workspace_bytes
         outs = 4 * sum(int(np.prod(s)) for s in self.output_shapes)
@@ -171,7 +186,9 @@ class HIPExecutable:
         self.arena = torch.empty(max(arena_bytes, 256), dtype=torch.uint8, device=self.device)
         # every split-K launch writes all the partials it reads: no clearing
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=self.device) if ws else None
-        self.constants = [torch.from_numpy(h).to(self.device) for h in host]
+        self.constants = [torch.from_numpy(h).to(self.device) if h is not None
+                          else pair_constant(program.derived[name], constants, name, self.device)
+                          for name, h in zip(program.consts, host)]
         self.plan.bind([c.data_ptr() for c in self.constants], self.arena.data_ptr(),
                        self.workspace.data_ptr() if ws else None, ws)
         self.guards = None

@@ -24,6 +24,7 @@ def interpreting(monkeypatch):
 
 def decode(copy, scales):
     b, n, kp = copy.shape
+    copy, scales = copy.numpy(), scales.numpy()
     h = copy.view(np.float16).reshape(b, n, kp // 8, 2, 8).astype(np.float64)
     return (h[:, :, :, 0] + h[:, :, :, 1]).reshape(b, n, kp) * scales.astype(np.float64)[:, :, None]
 
@@ -42,7 +43,7 @@ def test_pair_copy_holds_23_bits_per_column(k, n):
     top = np.abs(w).max(axis=0)
     assert (np.abs(got - w) <= 2.0 ** -23 * np.abs(w) + 2.0 ** -39 * top).all()
     assert (f16.pair_rows(*args).reshape(n, -1)[:, f16.padded_k(k):] == 0).all()
-    assert np.array_equal(f16.column_scales(*args, 5), f16.column_scales(*args, 0) / 32)
+    assert torch.equal(f16.column_scales(*args, 5), f16.column_scales(*args, 0) / 32)
 
 
 def _bounds(model, x):

@@ -73,6 +73,15 @@ def test_every_pair_configuration(tile):
             assert torch.equal(c(*args), out)
 
 
+def test_pair_copies_made_on_the_gpu_have_the_cpus_bits():
+    from kiln.hip import f16
+
+    w = np.random.default_rng(0).standard_normal((77, 133)).astype(np.float32) * np.logspace(-9, 5, 133, dtype=np.float32)
+    args = (w, 0, (0, 133, 1), 1, 77, 133)
+    assert torch.equal(f16.pair_rows(*args, "cuda").cpu(), f16.pair_rows(*args))
+    assert torch.equal(f16.column_scales(*args, 3, "cuda").cpu(), f16.column_scales(*args, 3))
+
+
 def test_columns_of_very_different_size_keep_their_precision():
     torch.manual_seed(3)
     model = _LnLinear(256, 96, "linear").eval()
