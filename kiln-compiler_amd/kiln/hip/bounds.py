@@ -1,12 +1,29 @@
-"""Upper bounds on activations, known at compile time.
+"""How large activations can be, and how large they usually are.
 
-An fp32 product runs on fp16 pairs (csrc/kh_gemm_f16.hip) only where its
-activations have a bound that holds for every input of the graph: their fixed
-power-of-two scale then never overflows fp16. In a pre-LN transformer every
-product has one: a LayerNorm's output is at most sqrt(C) max|gamma| + max|beta|
-whatever its input, a product with constant weights at most (row norm of its
-input) * (largest column norm of the weights), attention's output at most the
-largest |v|, and GELU, ReLU, tanh do not enlarge. A graph input has none.
+An fp32 product runs on fp16 pairs (csrc/kh_gemm_f16.hip) with one fixed power
+of two for all its activations, chosen at compile time. Two things are asked
+of it, both answered here from the graph and its constants:
+
+  * Safe: no value overflows fp16, whatever the input. That needs an upper
+    bound. In a pre-LN transformer every product has one: a LayerNorm's output
+    is at most sqrt(C) max|gamma| + max|beta| whatever its input, a product
+    with constant weights at most (row norm of its input) * (largest column
+    norm of the weights), attention's output at most the largest |v|, and GELU,
+    ReLU, tanh do not enlarge. A graph input has none.
+
+  * Tight: the values lie close enough under that bound. A pair holds 23 bits
+    of a value near the bound but has an absolute floor, PAIR_FLOOR of the
+    bound, and a bound grows by sqrt(N) per product that no LayerNorm follows,
+    or with one outlier gain, where the values do not. So beside the bound goes
+    each element's usual size: |gamma|, |beta| behind a LayerNorm (whose rows
+    have norm sqrt(C)), root sums of squares through products and additions,
+    half behind GELU and ReLU, a mean of `keys` independent values behind
+    attention. A product takes pairs only where, for every output column, the
+    floor stays a fraction of the rounding that fp32 operands of that size
+    bring anyway (2^-25 each); elsewhere it stays on the fp32 matrix cores. A
+    size is only claimed where it follows from the graph (an unknown one
+    refuses). Cancellation needs no care: what cancels has been rounded in fp32
+    before, relative to the terms.
 
 Bounds are for finite values: a NaN stays a NaN in fp16, and no infinity
 arises within a finite bound (a non-finite constant gives no bound).
@@ -15,30 +32,80 @@ arises within a finite bound (a non-finite constant gives no bound).
 from __future__ import annotations
 
 import math
+from dataclasses import dataclass
 
 import torch
 
-from kiln.hip import lib as kl
+from kiln.hip import f16
 
 NONE = (math.inf, math.inf)   # (largest magnitude, largest L2 norm of a row along the last dim)
 
+# Rounding of fp32 operands (2^-25 of a value, root mean square about half
+# that), and what a pair adds below its 23 bits: of an activation
+# PAIR_FLOOR of the bound, of a weight WEIGHT_FLOOR of its column's largest.
+FP32_ROUNDING = 2.0 ** -25
+PAIR_FLOOR = 2.0 ** -39
+WEIGHT_FLOOR = 2.0 ** -39
+# The floor's share of that rounding that is let through. GPT-2 blocks of
+# 2048 tokens reach 0.05 (their output projection, behind attention); at 0.5
+# the product's error grows by an eighth at most.
+SHARE = 0.5
 
-def _up(x: float) -> float:
-    """x rounded up to a power of two (so plans depend on constants' values
-    through few distinct numbers)."""
-    return x if x == 0.0 or not math.isfinite(x) else 2.0 ** math.ceil(math.log2(x))
+
+@dataclass
+class _Product:
+    """A product with a constant: largest column norm of the weights, the
+    output's size, and whether fp16 pairs hold both operands."""
+
+    column_norm: float
+    size: torch.Tensor
+    tight: bool
 
 
 class Bounds:
-    """Bounds of a lowered graph's values. ``row_pattern(kernel)`` recognises a
-    LayerNorm kernel: (1/C factor of the variance, gamma, beta) or None."""
+    """Bounds and sizes of a lowered graph's values. ``layer_norm(kernel, v)``
+    recognises a LayerNorm kernel: (1/C factor of the variance, eps, gamma,
+    beta) or None; ``attention(kernel)`` the match of an attention kernel."""
 
-    def __init__(self, graph, layer_norm, attention_value):
+    def __init__(self, graph, layer_norm, attention):
         self.g = graph
         self.layer_norm = layer_norm
-        self.attention_value = attention_value
+        self.attention = attention
         self._known = {}
-        self._norms = {}
+        self._sizes = {}
+        self._products = {}
+
+    # -- what the lowering asks ------------------------------------------------------
+
+    def pair_product(self, mm):
+        """Exponent of the scale of matmul node mm's A operand if the product
+        can run on fp16 pairs (safe and tight), else None."""
+        e = f16.activation_exponent(self.largest(mm.inputs[0]))
+        if e is None:
+            return None
+        return e if self.product(mm).tight else None
+
+    def pair_attention(self, m):
+        """Exponents of the scales of q, k and v of attention match m if it can
+        run on fp16 pairs, else None. Scores are asked per head, as a dot
+        product's operands are; v per head and dimension."""
+        tops = [self.largest(v) for v in (m.q, m.k, m.v)]
+        exponents = tuple(f16.activation_exponent(top) for top in tops)
+        if None in exponents:
+            return None
+        q, k, v = (self.size(x) for x in (m.q, m.k, m.v))
+        if m.k_transposed:
+            k = k.transpose(-2, -1)
+        # (a row's usual size: the smallest where it differs over the tokens)
+        q, k, v = (x.amin(dim=-2) for x in (q, k, v))
+        dh = m.q.shape[-1]
+        q, k = (x.expand(*x.shape[:-1], dh) for x in (q, k))
+        limit = SHARE * FP32_ROUNDING / PAIR_FLOOR
+        noise = (q * k).norm(dim=-1)
+        ok = (tops[0] * k.norm(dim=-1) <= limit * noise).all() and (tops[1] * q.norm(dim=-1) <= limit * noise).all()
+        return exponents if bool(ok) and bool((tops[2] <= limit * v).all()) else None
+
+    # -- upper bounds ----------------------------------------------------------------
 
     def largest(self, v) -> float:
         return self.of(v)[0]
@@ -49,7 +116,7 @@ class Bounds:
             top, norm = self._of(v)
             norm = min(norm, top * math.sqrt(v.shape[-1] if v.type.rank else 1))
             top = min(top, norm)
-            self._known[v] = (_up(top), _up(norm)) if math.isfinite(top) else NONE
+            self._known[v] = (top, norm) if math.isfinite(top) else NONE
         return self._known[v]
 
     def _constant(self, v):
@@ -59,45 +126,46 @@ class Bounds:
         data = self.g.const_data(v)
         return None if data is None else torch.as_tensor(data, dtype=torch.float32)
 
-    def _column_norm(self, b) -> float:
-        """Largest L2 norm of a column (along K) of a [.., K, N] constant."""
-        if b not in self._norms:
-            node, perm = b.node, False
-            if node is not None and node.op == "transpose" and b.type.rank == 2:
-                node, perm = node.inputs[0].node, True
-            data = self._constant(node.out) if node is not None else None
-            self._norms[b] = float(torch.linalg.vector_norm(data, dim=-1 if perm else -2).max()) \
-                if data is not None and data.dim() >= 2 and data.numel() else math.inf
-        return self._norms[b]
+    def _norm_of(self, v):
+        """(1/C factor, eps, gamma, beta) if v is a LayerNorm kernel's output."""
+        kernel = self.g.kernel_of(v.node)
+        return self.layer_norm(kernel, v) if kernel is not None and kernel.kind == "reduction" else None
+
+    def _attention_of(self, node):
+        """The match of the attention whose second product `node` is, else None."""
+        kernel = self.g.kernel_of(node)
+        if kernel is None or kernel.kind != "attention" or [n for n in kernel.nodes if n.op == "matmul"][-1] is not node:
+            return None
+        m = self.attention(kernel)
+        return m if m is not None and node.inputs[1] is m.v else None
 
     def _of(self, v):
         node = v.node
         if node is None:
             return NONE
-        kernel = self.g.kernel_of(node)
-        if kernel is not None and kernel.kind == "attention":
-            value = self.attention_value(kernel, v)
-            return (self.largest(value), math.inf) if value is not None else NONE
-        if kernel is not None and kernel.kind == "reduction":
-            found = self.layer_norm(kernel, v)
-            if found is not None:
-                c2, gamma, beta = found
-                if not c2 > 0.0:
-                    return NONE
-                scale = 1.0 / math.sqrt(c2)   # |x - mean| / sqrt(c2 sum (x - mean)^2 + eps), and its row norm
-                gt = self.of(gamma)[0] if gamma is not None else 1.0
-                bt, bn = self.of(beta) if beta is not None else (0.0, 0.0)
-                return gt * scale + bt, gt * scale + bn
+        found = self._norm_of(v)
+        if found is not None:
+            c2, eps, gamma, beta = found
+            if not (c2 > 0.0 and eps >= 0.0):
+                return NONE
+            scale = 1.0 / math.sqrt(c2)   # |x - mean| / sqrt(c2 sum (x - mean)^2 + eps), and its row norm
+            gt = self.of(gamma)[0] if gamma is not None else 1.0
+            bt, bn = self.of(beta) if beta is not None else (0.0, 0.0)
+            return gt * scale + bt, gt * scale + bn
         op, ins = node.op, node.inputs
         if op == "const":
             data = self._constant(v)
             if data is None or not data.numel() or not bool(torch.isfinite(data).all()):
                 return NONE
             top = float(data.abs().max())
-            return top, float(torch.linalg.vector_norm(data, dim=-1).max()) if data.dim() else top
+            rows = data.double()
+            return top, float(torch.linalg.vector_norm(rows, dim=-1).max()) if data.dim() else top
         if op == "matmul":
+            m = self._attention_of(node)
+            if m is not None:   # a weighted mean of rows of v
+                return self.largest(m.v), math.inf
             a_norm = self.of(ins[0])[1]
-            return (a_norm * self._column_norm(ins[1]), math.inf) if math.isfinite(a_norm) else NONE
+            return (a_norm * self.product(node).column_norm, math.inf) if math.isfinite(a_norm) else NONE
         if op in ("neg", "copy", "relu", "gelu"):   # |gelu(x)| <= |x|
             return self.of(ins[0])
         if op in ("tanh", "sigmoid", "erf"):
@@ -116,3 +184,129 @@ class Bounds:
             same_rows = op == "reshape" and ins[0].shape[-1:] == v.shape[-1:]
             return top, norm if same_rows else math.inf
         return NONE
+
+    # -- usual sizes -----------------------------------------------------------------
+
+    def size(self, v) -> torch.Tensor:
+        """Usual magnitude of v's elements (float64, v's rank; a dim of 1 means
+        alike along it); NaN where none is claimed."""
+        if v not in self._sizes:
+            unknown = _unknown(v.type.rank)
+            self._sizes[v] = unknown
+            found = self._size(v)
+            self._sizes[v] = unknown if found is None or not bool(torch.isfinite(found).all()) else found
+        return self._sizes[v]
+
+    def _size(self, v):
+        node = v.node
+        if node is None:
+            return None
+        found = self._norm_of(v)
+        if found is not None:
+            _, _, gamma, beta = found
+            shape = [1] * (v.type.rank - 1) + [v.shape[-1]]
+            parts = [p.reshape(shape) if p.numel() == v.shape[-1] else p.amin()
+                     for p in (self.size(x) for x in (gamma, beta) if x is not None)]
+            gain = parts[0] if gamma is not None else torch.ones(shape, dtype=torch.float64)
+            return torch.hypot(gain, parts[-1]) if beta is not None else gain
+        op, ins = node.op, node.inputs
+        if op == "const":
+            data = self._constant(v)
+            return None if data is None else data.double().abs()
+        if op == "matmul":
+            m = self._attention_of(node)
+            if m is not None:
+                return self.size(m.v).amin(dim=-2, keepdim=True) / math.sqrt(m.v.shape[-2])
+            return self.product(node).size
+        if op in ("neg", "copy"):
+            return self.size(ins[0])
+        if op in ("relu", "gelu"):
+            return self.size(ins[0]) / 2
+        if op in ("tanh", "erf"):
+            s = self.size(ins[0])
+            return s / torch.hypot(s, torch.ones_like(s))
+        if op in ("add", "sub"):
+            return torch.hypot(self.size(ins[0]), self.size(ins[1]))
+        if op == "mul" and any(self._constant(x) is not None for x in ins):
+            return self.size(ins[0]) * self.size(ins[1])
+        if op == "transpose":
+            return self.size(ins[0]).permute(node.attrs["perm"])
+        if op == "expand":
+            s = self.size(ins[0])
+            return s.reshape([1] * (v.type.rank - s.dim()) + list(s.shape))
+        if op == "slice":
+            s, dim = self.size(ins[0]), node.attrs["dim"] % v.type.rank
+            if s.shape[dim] == 1:
+                return s
+            index = torch.arange(node.attrs["start"], node.attrs["end"], node.attrs.get("step", 1))
+            return s.index_select(dim, index) if index.numel() == v.shape[dim] else None
+        if op == "reshape":
+            return _reshaped(self.size(ins[0]), ins[0].shape, v.shape)
+        return None
+
+    # -- products with constants -----------------------------------------------------
+
+    def product(self, mm) -> _Product:
+        if mm not in self._products:
+            self._products[mm] = self._product(mm)
+        return self._products[mm]
+
+    def _product(self, mm) -> _Product:
+        a, b = mm.inputs
+        rank = mm.out.type.rank
+        none = _Product(math.inf, _unknown(rank), False)
+        node, perm = b.node, False
+        if node is not None and node.op == "transpose" and b.type.rank == 2:
+            node, perm = node.inputs[0].node, True
+        w = self._constant(node.out) if node is not None else None
+        if w is None or w.dim() < 2 or not w.numel():
+            return none
+        w = w.transpose(-2, -1) if perm else w   # [.., K, N]
+        # columns scaled by their largest weight, so that squares neither
+        # overflow nor vanish; root sums of squares of the columns, plain and
+        # weighted by A's sizes, from one pass over the squares
+        top = torch.maximum(w.amax(dim=-2), -w.amin(dim=-2)).double()
+        if not bool(torch.isfinite(top).all()):
+            return none
+        unit = torch.where(top > 0, top, torch.ones_like(top))
+        # the smallest size along the other dims, for every K
+        s = self.size(a)
+        while s.dim() > 1:
+            s = s.amin(dim=0)
+        s = s.expand(w.shape[-2])
+        s_top = float(s.max()) or 1.0
+        squares = (w / unit.float().unsqueeze(-2)).square_()
+        weighted = torch.stack([torch.ones_like(s), (s / s_top).square()]).float() @ squares   # [.., 2, N]
+        norm = top * weighted[..., 0, :].double().sqrt()
+        noise = top * s_top * weighted[..., 1, :].double().sqrt()
+        bound = self.largest(a)
+        tight = bool((bound * norm * PAIR_FLOOR <= SHARE * FP32_ROUNDING * noise).all()) and bool(
+            (top * float(s.norm()) * WEIGHT_FLOOR <= SHARE * FP32_ROUNDING * noise).all()) and f16.columns_fit(top)
+        size = noise.unsqueeze(-2) if noise.dim() > 1 else noise
+        return _Product(float(norm.max()), size.reshape([1] * (rank - size.dim()) + list(size.shape)), tight)
+
+
+def _unknown(rank):
+    return torch.full([1] * rank, math.nan, dtype=torch.float64)
+
+
+def _reshaped(s, old, new):
+    """Sizes `s` (of a value of shape `old`, dims of 1 where alike) as sizes of
+    the same value reshaped to `new`."""
+    if not all(old) or not all(new):
+        return None
+    source, target, i, j = [], [], 0, 0
+    while i < len(old) or j < len(new):
+        # the next groups of dims with the same number of elements
+        i0, j0 = i, j
+        a, b = (old[i] if i < len(old) else 1), (new[j] if j < len(new) else 1)
+        i, j = min(i + 1, len(old)), min(j + 1, len(new))
+        while a != b:
+            if a < b:
+                a, i = a * old[i], i + 1
+            else:
+                b, j = b * new[j], j + 1
+        alike = all(s.shape[d] == 1 for d in range(i0, i))
+        source += [1] * (i - i0) if alike else list(old[i0:i])
+        target += [1] * (j - j0) if alike else list(new[j0:j])
+    return s.expand(source).reshape(target)

@@ -54,6 +54,13 @@ def row_exponents(rows: torch.Tensor) -> torch.Tensor:
     return torch.where(top > 0, TOP + 1 - exponent, torch.zeros_like(exponent)).clamp(*WEIGHT_EXPONENTS)
 
 
+def columns_fit(top: torch.Tensor) -> bool:
+    """Is no column's power of two (largest weights ``top``) out of range?"""
+    _, exponent = torch.frexp(top[top > 0])
+    e = TOP + 1 - exponent
+    return not e.numel() or (int(e.min()) >= WEIGHT_EXPONENTS[0] and int(e.max()) <= WEIGHT_EXPONENTS[1])
+
+
 def _power_of_two(e: torch.Tensor) -> torch.Tensor:
     """float32 2^e, |e| <= 126, from its bits (torch.ldexp goes through pow,
     which the GPU does not round to an exact power)."""

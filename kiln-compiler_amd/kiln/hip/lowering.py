@@ -214,7 +214,7 @@ class _Lowerer:
         self.bf16_buffers = set()   # arena buffers held as bf16 (plan_bf16_storage)
         self.pair_buffers = set()   # arena buffers held as pair words (plan_pair_storage)
         self.f16_buffers = {}       # arena buffers held as fp16 pairs -> exponent of their scale (plan_f16_storage)
-        self.bounds = Bounds(graph, self._layer_norm_of, self._attention_value_of)
+        self.bounds = Bounds(graph, self._layer_norm_of, self._attention_match)
         self.precision = precision
         self.matmul_config = matmul_config
         self.program = Program(precision=precision)
@@ -424,8 +424,11 @@ class _Lowerer:
         if (strides is None or m.q.shape[1] <= ATTN_ROWS_MAX_Q or ATTN_QUERIES == 16
                 or m.v.shape[1] < ATTN_F16_MIN_KEYS):
             return None
+        exponents = self.bounds.pair_attention(m)
+        if exponents is None:
+            return None
         out = {}
-        for v, (offset, st) in zip((m.q, m.k, m.v), strides):
+        for v, (offset, st), e in zip((m.q, m.k, m.v), strides, exponents):
             lay = self.layouts.get(v)
             if lay is None or lay.base[0] != "arena" or offset % 8 or st[0] % 8 or st[1] % 8:
                 return None
@@ -434,8 +437,7 @@ class _Lowerer:
             if (self._arena_readers().get(buf) != {k} or buf in self.g.results or producer is None
                     or producer.kind != "matmul"):
                 return None
-            e = f16.activation_exponent(self.bounds.largest(buf))
-            if e is None or not self._writes_f16(producer, buf):
+            if out.get(buf, e) != e or not self._writes_f16(producer, buf):
                 return None
             out[buf] = e
         return out
@@ -467,10 +469,8 @@ class _Lowerer:
         producer = self.g.kernel_of(buf.node)
         if producer is None or not self._writes_f16(producer, buf):
             return None
-        e = f16.activation_exponent(self.bounds.largest(a))
-        if e is None or not math.isfinite(self.bounds._column_norm(b)):
-            return None
-        return buf, e
+        e = self.bounds.pair_product(mm)
+        return None if e is None else (buf, e)
 
     def _writes_f16(self, k, buf) -> bool:
         """Can kernel k write its output `buf` as fp16 pairs? The one-wave
@@ -493,8 +493,8 @@ class _Lowerer:
         return (prec == "f16x3" or small) and self._bias_act_epilogue(k, buf)
 
     def _layer_norm_of(self, k, v):
-        """(factor of the variance's sum, gamma, beta) if v is the output of a
-        LayerNorm kernel k, else None."""
+        """(factor of the variance's sum, eps, gamma, beta) if v is the output
+        of a LayerNorm kernel k, else None."""
         reds = [n for n in k.nodes if n.op.startswith("reduce_")]
         outs = kernel_outputs(self.g, k, self.users)
         if outs != [v] or not reds or not all(is_row_reduction(n) for n in reds):
@@ -502,7 +502,7 @@ class _Lowerer:
         variant, fparams, (has_g, has_b), ordered = self._row_pattern(k, reds, outs, self._externals(k))
         if variant != kl.ROW_LAYERNORM or ordered is None:
             return None
-        return fparams[1], ordered[1] if has_g else None, ordered[1 + has_g] if has_b else None
+        return fparams[1], fparams[2], ordered[1] if has_g else None, ordered[1 + has_g] if has_b else None
 
     def _one_wave_rows(self, k, buf) -> bool:
         """Does LayerNorm kernel k (out buf) meet the library's conditions for
@@ -527,12 +527,10 @@ class _Lowerer:
                     out.append(v)
         return out
 
-    def _attention_value_of(self, k, v):
-        """The V operand of attention kernel k if v is its result, else None."""
+    def _attention_match(self, k):
         from kiln.hip.attention import match_kernel
 
-        m = match_kernel(self.g, k)
-        return m.v if m is not None and (v is m.result or v in kernel_outputs(self.g, k, self.users)) else None
+        return match_kernel(self.g, k)
 
     def _bias_act_epilogue(self, k, buf) -> bool:
         """Is matmul kernel k's tape out = act(acc + bias), act none, GELU or

@@ -2,6 +2,8 @@
 bounds that make a fixed activation scale safe, which products take the path,
 and the plan's meaning through the host interpreter."""
 
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -72,6 +74,20 @@ def test_bounds_hold_whatever_the_input(scale):
     assert float(ln(x).abs().max()) > tops[0] / 64   # not vacuous
     for top in tops:
         assert top * 2.0 ** f16.activation_exponent(top) <= 2.0 ** f16.TOP
+
+
+class SelfAttention(torch.nn.Module):
+    """LayerNorm -> q, k, v (one product) -> attention, heads merged."""
+
+    def __init__(self, d, heads):
+        super().__init__()
+        self.heads, self.ln, self.qkv = heads, torch.nn.LayerNorm(d), torch.nn.Linear(d, 3 * d)
+
+    def forward(self, x):
+        t, c = x.shape
+        q, k, v = (y.view(t, self.heads, c // self.heads).transpose(0, 1) for y in self.qkv(self.ln(x)).split(c, dim=1))
+        y = F.softmax((q @ k.transpose(-2, -1)) * 0.125, dim=-1) @ v
+        return y.transpose(0, 1).contiguous().view(t, c)
 
 
 def test_bounds_refuse_what_has_none():
@@ -155,3 +171,120 @@ def test_callers_configuration_on_pairs():
         prog = lower_graph(g, matmul_config=cfg)
         assert (f"tile {tile} splitk 1 f16x3" in prog.launches[-1].summary) == on_pairs
     assert autotune.PRECISION[tile] == "f16x3"
+
+
+# -- products whose bound lies far above their values -----------------------------------------
+
+
+def _chain(n, width, activation, kaiming):
+    layers = [torch.nn.LayerNorm(width)]
+    for _ in range(n):
+        lin = torch.nn.Linear(width, width)
+        if kaiming:
+            torch.nn.init.kaiming_normal_(lin.weight, nonlinearity="relu")
+        layers += [lin] + ([activation()] if activation else [])
+    return torch.nn.Sequential(*layers, torch.nn.Linear(width, width)).eval()
+
+
+def _errors(model, x):
+    """Relative errors against float64 of the compiled model and of eager
+    fp32, and the number of products on pairs."""
+    c = kiln.compile(model, (x,), device="cuda")
+    with torch.no_grad():
+        got, eager, ref = c(x).double(), model(x).double(), copy.deepcopy(model).double()(x.double())
+    pairs = sum("f16x3" in l.summary for l in c._exe.program.launches)
+    return *(float((t - ref).norm() / ref.norm()) for t in (got, eager)), pairs
+
+
+@pytest.mark.parametrize("activation,kaiming", [(torch.nn.GELU, False), (torch.nn.ReLU, True), (None, False)])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 8, 10, 12])
+def test_deep_chains_are_as_precise_as_eager(interpreting, n, activation, kaiming):
+    # the bound grows by sqrt(width) per product, the values do not: products
+    # far from the LayerNorm stay off pairs (on pairs: 0.3 to 1.0 at n = 10)
+    torch.manual_seed(n)
+    err, eager, pairs = _errors(_chain(n, 64, activation, kaiming), torch.randn(40, 64))
+    assert err <= eager
+    assert 1 <= pairs <= 4
+
+
+@pytest.mark.parametrize("outlier", [1e2, 1e4, 1e6, 1e12])
+@pytest.mark.parametrize("where", ["gain", "unused gain", "weight", "hidden column"])
+def test_outliers_keep_the_other_values_precise(interpreting, outlier, where):
+    # one gain, weight or hidden column of another size, taken back by what
+    # follows it: it sets the scale that all the others share
+    torch.manual_seed(0)
+    ln, fc, proj = torch.nn.LayerNorm(64), torch.nn.Linear(64, 64), torch.nn.Linear(64, 64)
+    with torch.no_grad():
+        if where == "gain":
+            ln.weight[0] = outlier
+            fc.weight[:, 0] /= outlier
+        elif where == "unused gain":
+            ln.weight[0] = outlier
+            fc.weight[:, 0] = 0.0
+        elif where == "weight":
+            ln.weight[0] = 0.1 / outlier
+            fc.weight[:, 0] *= outlier
+        else:
+            fc.weight[0] *= outlier
+            proj.weight[:, 0] /= outlier
+    err, eager, _ = _errors(torch.nn.Sequential(ln, fc, proj).eval(), torch.randn(300, 64))
+    assert err <= eager
+
+
+def test_columns_out_of_the_scales_range_stay_off_pairs(interpreting):
+    # a column's power of two is clamped: weights below 2^-66 would be fp16
+    # subnormals. And bounds whose squares vanish in fp32 are still bounds.
+    torch.manual_seed(0)
+    ln, fc, proj = torch.nn.LayerNorm(64), torch.nn.Linear(64, 64, bias=False), torch.nn.Linear(64, 64)
+    with torch.no_grad():
+        fc.weight *= 1e-25
+    err, eager, pairs = _errors(torch.nn.Sequential(ln, fc).eval(), torch.randn(300, 64))
+    assert err <= eager and pairs == 0
+    with torch.no_grad():
+        ln.weight *= 1e24
+    g, low = _bounds(torch.nn.Sequential(ln, fc, proj).eval(), torch.randn(300, 64))
+    mm = [n for n in g.nodes if n.op == "matmul"][-1]
+    with torch.no_grad():
+        hidden = fc(ln(torch.randn(300, 64)))
+    assert float(hidden.abs().max()) <= low.bounds.largest(mm.inputs[0]) < float("inf")
+
+
+@pytest.mark.parametrize("scale_q,scale_v,on_pairs", [(1.0, 1.0, True), (64.0, 8.0, True), (1e5, 1.0, False),
+                                                      (1.0, 1e-5, False)])
+def test_attention_on_pairs_needs_tight_bounds(scale_q, scale_v, on_pairs):
+    # a head of another size shares the others' scale
+    torch.manual_seed(0)
+    model = SelfAttention(128, 2).eval()
+    with torch.no_grad():
+        model.qkv.weight[:64] *= scale_q
+        model.qkv.weight[256 + 64:] *= scale_v
+        model.qkv.bias[:64] *= scale_q
+        model.qkv.bias[256 + 64:] *= scale_v
+    g, prog = lowered(model, torch.randn(200, 128), fuse_attention=True)
+    assert any("products:f16x3" in l.summary for l in prog.launches) == on_pairs
+
+
+@pytest.mark.parametrize("T,d,heads", [(512, 768, 12), (2048, 768, 12), (2048, 1024, 16), (333, 128, 4)])
+def test_blocks_are_tight(T, d, heads):
+    # the bounds of a block lie close enough for all its products and attention
+    g, prog = lowered(gpt2_init_(Block(d, heads, T), seed=0), torch.randn(T, d), fuse_attention=True)
+    assert sum("f16x3" in l.summary for l in prog.launches) == 5
+
+
+def test_sizes_follow_the_graph():
+    # measured rows against the sizes the gate works with: a LayerNorm's per
+    # column, through a product, GELU, views and attention to a small factor
+    torch.manual_seed(0)
+    model = SelfAttention(128, 2).eval()
+    with torch.no_grad():
+        model.ln.weight.uniform_(0.2, 3.0), model.ln.bias.uniform_(-0.5, 0.5)
+    x = torch.randn(200, 128)
+    g, low = _bounds(model, x)
+    (kernel,) = [k for k in g.kernels if k.kind == "attention"]
+    m = low._attention_match(kernel)
+    with torch.no_grad():
+        q, k, v = (t.view(200, 2, 64).transpose(0, 1) for t in model.qkv(model.ln(x)).split(128, dim=1))
+    for value, data in ((m.q, q), (m.v, v)):
+        ratio = data.double().square().mean(dim=-2, keepdim=True).sqrt() / low.bounds.size(value)
+        assert ratio.shape == (2, 1, 64) and 0.7 < float(ratio.min()) and float(ratio.max()) < 1.4
+    assert torch.isnan(low.bounds.size(g.args[0])).all()
