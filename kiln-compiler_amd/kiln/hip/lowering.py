@@ -343,7 +343,7 @@ class _Lowerer:
         if lay is None or lay.base[0] != "arena" or lay.offset != 0 or lay.strides[-1] != 1:
             return None
         buf = lay.base[1]
-        if self._arena_readers().get(buf) != {k} or buf in self.g.results:
+        if not self._reads_only(k, buf, [a]) or buf in self.g.results:
             return None
         producer = self.g.kernel_of(buf.node)
         return buf if producer is not None and self._writes_pairs(producer, buf) else None
@@ -368,7 +368,7 @@ class _Lowerer:
         if len(bufs) != 1:
             return None
         buf = bufs.pop()
-        if self._arena_readers().get(buf) != {k} or buf in self.g.results:
+        if not self._reads_only(k, buf, [m.q, m.k, m.v]) or buf in self.g.results:
             return None
         producer = self.g.kernel_of(buf.node)
         return buf if producer is not None and producer.kind == "matmul" and self._writes_pairs(producer, buf) else None
@@ -434,7 +434,7 @@ class _Lowerer:
                 return None
             buf = lay.base[1]
             producer = self.g.kernel_of(buf.node)
-            if (self._arena_readers().get(buf) != {k} or buf in self.g.results or producer is None
+            if (not self._reads_only(k, buf, [m.q, m.k, m.v]) or buf in self.g.results or producer is None
                     or producer.kind != "matmul"):
                 return None
             if out.get(buf, e) != e or not self._writes_f16(producer, buf):
@@ -464,7 +464,8 @@ class _Lowerer:
                 st % 8 for st, ext in zip(lay.strides[:-1], lay.shape[:-1]) if ext > 1):
             return None
         buf = lay.base[1]
-        if buf.type.nbytes != 4 * math.prod(a.shape) or self._arena_readers().get(buf) != {k} or buf in self.g.results:
+        if (buf.type.nbytes != 4 * math.prod(a.shape) or not self._reads_only(k, buf, [a])
+                or buf in self.g.results):
             return None
         producer = self.g.kernel_of(buf.node)
         if producer is None or not self._writes_f16(producer, buf):
@@ -561,6 +562,21 @@ class _Lowerer:
                             self._readers.setdefault(lay.base[1], set()).add(k)
         return self._readers
 
+    def _reads_only(self, k, buf, operands):
+        """Does kernel k alone read arena buffer buf, and only as `operands`,
+        each in one place? (An epilogue or a mask reads fp32: a product's A
+        operand that is its residual too cannot be stored another way.)"""
+        if self._arena_readers().get(buf) != {k}:
+            return False
+        members = set(k.nodes)
+        places = {}
+        for n in k.nodes:
+            for v in n.inputs:
+                lay = self.layouts.get(v)
+                if lay is not None and lay.base == ("arena", buf) and v.node not in members:
+                    places[v] = places.get(v, 0) + 1
+        return set(places) <= set(operands) and all(n == operands.count(v) for v, n in places.items())
+
     def a16_buffer(self, k):
         """The arena buffer of matmul kernel k's A operand if it can be stored
         as bf16 for a product that reads A that way: A is the whole buffer,
@@ -580,7 +596,7 @@ class _Lowerer:
         buf = lay.base[1]
         if a.shape[-1] % 8 or any(st % 8 for st, ext in zip(lay.strides[:-1], lay.shape[:-1]) if ext > 1):
             return None
-        if self._arena_readers().get(buf) != {k} or buf in self.g.results:
+        if not self._reads_only(k, buf, [a]) or buf in self.g.results:
             return None
         producer = self.g.kernel_of(buf.node)
         return buf if producer is not None and self._rounds_to_bf16(producer, buf) else None
@@ -608,7 +624,7 @@ class _Lowerer:
         if len(bufs) != 1:
             return None
         buf = bufs.pop()
-        if self._arena_readers().get(buf) != {k} or buf in self.g.results:
+        if not self._reads_only(k, buf, [m.q, m.k, m.v]) or buf in self.g.results:
             return None
         producer = self.g.kernel_of(buf.node)
         return buf if producer is not None and producer.kind == "matmul" and self._rounds_to_bf16(producer, buf) else None

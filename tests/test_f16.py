@@ -288,3 +288,32 @@ def test_sizes_follow_the_graph():
         ratio = data.double().square().mean(dim=-2, keepdim=True).sqrt() / low.bounds.size(value)
         assert ratio.shape == (2, 1, 64) and 0.7 < float(ratio.min()) and float(ratio.max()) < 1.4
     assert torch.isnan(low.bounds.size(g.args[0])).all()
+
+
+# -- storage of operands that are read another way too ------------------------------------------
+
+
+class _ResidualOnNorm(torch.nn.Module):
+    """y + W y of y = LayerNorm(x): the product's A operand is its residual."""
+
+    def __init__(self, d, view):
+        super().__init__()
+        self.ln, self.lin, self.view = torch.nn.LayerNorm(d), torch.nn.Linear(d, d), view
+
+    def forward(self, x):
+        y = self.ln(x)
+        if self.view:   # the residual through a view of the same buffer
+            return self.lin(y) + y.view(2, x.shape[0] // 2, -1).transpose(0, 1).transpose(0, 1).reshape(x.shape)
+        return self.lin(y) + y
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "bf16x3"])
+@pytest.mark.parametrize("T,d,tile", [(300, 64, None), (600, 64, None), (600, 256, 98), (40, 64, None)])
+@pytest.mark.parametrize("view", [False, True])
+def test_operand_that_is_also_the_residual_stays_fp32(interpreting, precision, T, d, tile, view):
+    torch.manual_seed(0)
+    cfg = {"gpu_matmul_config": lambda *_: {"tile": tile, "splitk": 1}} if tile is not None and precision == "bf16" else {}
+    c = check(_ResidualOnNorm(d, view).eval(), torch.randn(T, d), matmul_precision=precision, **cfg,
+              **({} if precision == "fp32" else {"rtol": 2e-2, "atol": 2e-2}))
+    product = c._exe.program.launches[-1].desc
+    assert product.cfg[7] & 1 == 0 and product.cfg[7] >> 16 & 1 == 0

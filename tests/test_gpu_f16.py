@@ -186,3 +186,15 @@ def test_block_on_pairs(T):
     exe._static[0][0].copy_(x.cuda())
     exe.replay_only()
     assert torch.equal(exe._static[1][0], c(x.cuda()))
+
+
+@pytest.mark.parametrize("precision,tol", [("fp32", 1e-4), ("bf16x3", 1e-4), ("bf16", 2e-2)])
+def test_operand_that_is_also_the_residual(precision, tol):
+    from test_f16 import _ResidualOnNorm
+
+    torch.manual_seed(0)
+    model, x = _ResidualOnNorm(256, False).eval(), torch.randn(600, 256)
+    out = kiln.compile(model, (x,), device="cuda", matmul_precision=precision)(x.cuda()).cpu()
+    with torch.no_grad():
+        ref = model.double()(x.double())
+    np.testing.assert_allclose(out.double().numpy(), ref.numpy(), rtol=tol, atol=tol)
