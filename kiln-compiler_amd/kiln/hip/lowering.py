@@ -1760,14 +1760,18 @@ class _Lowerer:
 
 
 def operand_scales(graph: Graph) -> str:
-    """The exponents that fp16 pairs could scale the graph's products by: what
-    an fp32 plan depends on of the constants' values."""
+    """What an fp32 plan takes from the constants' values, as text: for every
+    product the exponent of the scale its A operand could be stored with as
+    fp16 pairs, for every attention those of q, k and v, None where values and
+    bounds keep it off pairs. The lowering asks the same two questions."""
     low = _Lowerer(graph, "fp32", None)
     out = []
     for k in graph.kernels:
         if k.kind == "matmul":
-            mm = next(n for n in k.nodes if n.op == "matmul")
-            out.append(f16.activation_exponent(low.bounds.largest(mm.inputs[0])))
+            out.append(low.bounds.pair_product(next(n for n in k.nodes if n.op == "matmul")))
+        elif k.kind == "attention":
+            m = low._attention_match(k)
+            out.append(low.bounds.pair_attention(m) if m is not None else None)
     return repr(out)
 
 

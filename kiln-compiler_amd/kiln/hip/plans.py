@@ -12,10 +12,11 @@ lowering and tuner sources, the shipped tuning table, the library's ABI
 version, struct sizes and GEMM configuration table), the device (arch, CU
 count), the matmul precision, how GEMM configurations were chosen, and the
 optimised graph's text (ops, shapes, kernel partition, buffer layouts and
-arena offsets). Constant *data* is part of it only through the powers of two
-that fp32 products on fp16 pairs scale their operands by (the caller adds
-them to ``config_source``): no other descriptor depends on it, derived copies
-are rebuilt from the recipes.
+arena offsets). Constant *data* is part of it only through what the lowering
+takes from it (lowering.operand_scales, which the caller adds to
+``config_source``): the powers of two that fp32 products and attention on fp16
+pairs scale their operands by, and which of them stay off pairs. Derived
+copies are rebuilt from the recipes.
 
 Files live in ``<cache dir>/plans/<key>.json`` (written to a temporary file,
 flushed, then renamed, so a crash never leaves a half-written plan behind),

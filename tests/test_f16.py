@@ -317,3 +317,53 @@ def test_operand_that_is_also_the_residual_stays_fp32(interpreting, precision, T
               **({} if precision == "fp32" else {"rtol": 2e-2, "atol": 2e-2}))
     product = c._exe.program.launches[-1].desc
     assert product.cfg[7] & 1 == 0 and product.cfg[7] >> 16 & 1 == 0
+
+
+# -- stored plans -------------------------------------------------------------------------------
+
+
+class _Projected(SelfAttention):
+    """SelfAttention with separate q, k and v products and an output projection."""
+
+    def __init__(self, d, heads):
+        super().__init__(d, heads)
+        self.q, self.k, self.v, self.proj = (torch.nn.Linear(d, d) for _ in range(4))
+
+    def forward(self, x):
+        t, c = x.shape
+        y = self.ln(x)
+        q, k, v = (f(y).view(t, self.heads, c // self.heads).transpose(0, 1) for f in (self.q, self.k, self.v))
+        y = F.softmax((q @ k.transpose(-2, -1)) * 0.125, dim=-1) @ v
+        return self.proj(y.transpose(0, 1).contiguous().view(t, c))
+
+
+def _descs(program):
+    return [bytes(l.desc) for l in program.launches]
+
+
+@pytest.mark.parametrize("change", [
+    ("qkv", 4096.0), ("qkv", 2.0 ** -12), ("one head", 1e6), ("q", 4096.0), ("v", 4096.0), ("v", 2.0 ** -12),
+    ("column", 1e-25)])
+def test_stored_plan_is_not_reused_with_other_scales(interpreting, tmp_path, monkeypatch, change):
+    # two models of one structure against one cache: the second's plan has
+    # the scales, and the storage, that a fresh lowering gives it
+    monkeypatch.setenv("KILN_CACHE_DIR", str(tmp_path))
+    what, factor = change
+    torch.manual_seed(0)
+    model = (_Projected if what in ("q", "v", "column") else SelfAttention)(64, 2 if what != "qkv" else 1).eval()
+    x = torch.randn(192, 64)
+    first = kiln.compile(model, (x,), device="cuda")
+    assert any("products:f16x3" in l.summary for l in first._exe.program.launches)
+    again = kiln.compile(model, (x,), device="cuda")
+    assert again.report.lowering["plan_cache"] == "stored"
+    with torch.no_grad():
+        if what == "one head":
+            model.qkv.weight[:32] *= factor
+        elif what == "column":
+            model.proj.weight[0] *= factor
+        else:
+            getattr(model, what).weight.mul_(factor)
+    second = kiln.compile(model, (x,), device="cuda")
+    fresh = kiln.compile(model, (x,), device="cuda", plan_cache=False)
+    assert _descs(second._exe.program) == _descs(fresh._exe.program) != _descs(first._exe.program)
+    assert second.report.lowering["plan_cache"] == "lowered"
