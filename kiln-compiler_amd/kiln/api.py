@@ -192,8 +192,7 @@ class _GpuBuild:
             source = source_name + "|gemv-chains" if self.options.gemv_chains else source_name
             if lowering.ATTN_QUERIES:
                 source += f"|attention-q{lowering.ATTN_QUERIES}"
-            if self.precision == "fp32":
-                source += "|scales " + lowering.operand_scales(self.graph)
+            source += "|" + lowering.constant_facts(self.graph, self.precision)
             key = plans.plan_key(str(self.graph), self.precision, source, kl.device_info())
             stored = plans.load(key)
             if stored is not None:

@@ -267,8 +267,6 @@ def causal_or_none(graph: Graph, mask, batch, tq, tk):
         return None
     data = np.asarray(graph.const_data(mask), dtype=np.float32)
     full = np.broadcast_to(data.reshape(mask.shape), (batch, tq, tk) if mask.type.rank == 3 else (tq, tk))
-    i = np.arange(tq)[:, None]
-    j = np.arange(tk)[None, :]
-    above = np.broadcast_to(j > i, (tq, tk))
-    ok = np.all(np.isneginf(full[..., above])) and np.all(full[..., ~above] == 0.0)
+    want = np.triu(np.full((tq, tk), -np.inf, np.float32), 1)
+    ok = np.array_equal(full, np.broadcast_to(want, full.shape))
     return kl.ATTN_MASK_CAUSAL if ok else None

@@ -1775,6 +1775,20 @@ def operand_scales(graph: Graph) -> str:
     return repr(out)
 
 
+def constant_facts(graph: Graph, precision: str) -> str:
+    """What a plan takes from the constants' values, as text: which attention
+    masks are the causal one, and an fp32 plan's operand scales."""
+    from kiln.hip.attention import causal_or_none, match_kernel
+
+    masks = []
+    for k in graph.kernels:
+        m = match_kernel(graph, k) if k.kind == "attention" else None
+        if m is not None:
+            batch, tq, _ = m.q.shape
+            masks.append(causal_or_none(graph, m.mask, batch, tq, m.v.shape[1]))
+    return f"masks {masks}" + (f" scales {operand_scales(graph)}" if precision == "fp32" else "")
+
+
 def lower_graph(graph: Graph, precision: str = "fp32", matmul_config=None, gemv_chains: bool = False) -> Program:
     """Fused, buffer-assigned, memory-planned graph -> Program (launch list).
     gemv_chains: mark one-row matmuls KH_GEMV_CHAIN, so the library may run

@@ -13,10 +13,10 @@ version, struct sizes and GEMM configuration table), the device (arch, CU
 count), the matmul precision, how GEMM configurations were chosen, and the
 optimised graph's text (ops, shapes, kernel partition, buffer layouts and
 arena offsets). Constant *data* is part of it only through what the lowering
-takes from it (lowering.operand_scales, which the caller adds to
-``config_source``): the powers of two that fp32 products and attention on fp16
-pairs scale their operands by, and which of them stay off pairs. Derived
-copies are rebuilt from the recipes.
+takes from it (lowering.constant_facts, which the caller adds to
+``config_source``): which attention masks are causal, the powers of two that
+fp32 products and attention on fp16 pairs scale their operands by, and which
+of them stay off pairs. Derived copies are rebuilt from the recipes.
 
 Files live in ``<cache dir>/plans/<key>.json`` (written to a temporary file,
 flushed, then renamed, so a crash never leaves a half-written plan behind),

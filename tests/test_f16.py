@@ -367,3 +367,31 @@ def test_stored_plan_is_not_reused_with_other_scales(interpreting, tmp_path, mon
     fresh = kiln.compile(model, (x,), device="cuda", plan_cache=False)
     assert _descs(second._exe.program) == _descs(fresh._exe.program) != _descs(first._exe.program)
     assert second.report.lowering["plan_cache"] == "lowered"
+
+
+class _Masked(SelfAttention):
+    def __init__(self, d, heads, mask):
+        super().__init__(d, heads)
+        self.register_buffer("mask", mask)
+
+    def forward(self, x):
+        t, c = x.shape
+        q, k, v = (y.view(t, self.heads, c // self.heads).transpose(0, 1) for y in self.qkv(self.ln(x)).split(c, dim=1))
+        y = F.softmax(q @ k.transpose(-2, -1) * 0.2 + self.mask, dim=-1) @ v
+        return y.transpose(0, 1).contiguous().view(t, c)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16x3", "bf16"])
+@pytest.mark.parametrize("T", [1, 40])
+def test_stored_plan_is_not_reused_with_another_mask(interpreting, tmp_path, monkeypatch, precision, T):
+    # a causal mask is not read by its plan; another mask of the same shape is
+    monkeypatch.setenv("KILN_CACHE_DIR", str(tmp_path))
+    causal = torch.full((T, T), float("-inf")).triu(1)
+    x = torch.randn(T, 64)
+    for mask in (causal, torch.randn(T, T) if T > 1 else torch.full((1, 1), float("-inf")), causal):
+        torch.manual_seed(0)
+        model = _Masked(64, 2, mask).eval()
+        c = kiln.compile(model, (x,), device="cuda", matmul_precision=precision)
+        with torch.no_grad():
+            torch.testing.assert_close(c(x), model(x), rtol=3e-2, atol=3e-2, equal_nan=True)
+    assert c.report.lowering["plan_cache"] == "stored"
