@@ -22,6 +22,8 @@ TOP = 14
 # exponents that keep every scale and product of scales a normal float32
 WEIGHT_EXPONENTS = (-80, 80)
 ACTIVATION_EXPONENTS = (-40, 40)
+# elements of a pair copy that are made at a time (temporaries of ~100 MB)
+CHUNK = 4 << 20
 
 
 def activation_exponent(bound: float):
@@ -67,26 +69,59 @@ def _power_of_two(e: torch.Tensor) -> torch.Tensor:
     return ((e.int() + 127) << 23).view(torch.float32)
 
 
-def pair_rows(data, offset, strides, batch: int, k: int, n: int, device="cpu") -> torch.Tensor:
-    """The [batch, N, K'] pair copy (int32 words, on `device`) of the [batch, K,
-    N] view of a constant, each row times its own power of two (row_exponents).
-    The same bits on the CPU and on the GPU, where it is ~100 times faster."""
-    rows = _rows(data, offset, strides, batch, k, n, device)
-    rows = rows.contiguous() * _power_of_two(row_exponents(rows)).unsqueeze(-1)
+def column_exponents(data, offset, strides, batch: int, k: int, n: int, device="cpu") -> torch.Tensor:
+    """The exponents of the powers of two of the [batch, K, N] view's columns
+    (int32 [batch, N], on `device`)."""
+    return row_exponents(_rows(data, offset, strides, batch, k, n, device))
+
+
+def pair_rows(data, offset, strides, batch: int, k: int, n: int, device="cpu", chunk=CHUNK) -> torch.Tensor:
+    """The pair copy alone (see pair_copy)."""
+    return pair_copy(data, offset, strides, batch, k, n, device, chunk)[0]
+
+
+def pair_copy(data, offset, strides, batch: int, k: int, n: int, device="cpu", chunk=CHUNK):
+    """(the [batch, N, K'] pair copy (int32 words, on `device`) of the [batch, K,
+    N] view of a constant, each row times its own power of two; the exponents
+    of those, as column_exponents gives them). The same bits on the CPU and on
+    the GPU, where it is ~100 times faster. Made a few rows at a time, `chunk`
+    elements: beside the result and the constant itself it takes
+    scratch_bytes."""
+    source = _rows(data, offset, strides, batch, k, n, device)
     kp = padded_k(k)
-    if kp != k:
-        rows = torch.nn.functional.pad(rows, (0, kp - k))
-    rows = rows.view(batch, n, kp // 8, 8)
-    h = rows.half()   # (rounds to nearest)
-    l = (rows - h.float()).half()
-    return torch.stack([h, l], dim=3).view(torch.int32).view(batch, n, kp)
+    out = torch.empty((batch, n, kp // 8, 2, 8), dtype=torch.float16, device=device)
+    exponents = torch.empty((batch, n), dtype=torch.int32, device=device)
+    step = max(1, chunk // kp)
+    for b in range(batch):
+        for at in range(0, n, step):
+            rows = source[b, at:at + step].contiguous()
+            e = exponents[b, at:at + step] = row_exponents(rows)
+            rows = rows * _power_of_two(e).unsqueeze(-1)
+            if kp != k:
+                rows = torch.nn.functional.pad(rows, (0, kp - k))
+            rows = rows.view(-1, kp // 8, 8)
+            h = rows.half()   # (rounds to nearest)
+            out[b, at:at + step, :, 0] = h
+            out[b, at:at + step, :, 1] = (rows - h.float()).half()
+    return out.view(torch.int32).view(batch, n, kp), exponents
 
 
 def column_scales(data, offset, strides, batch: int, k: int, n: int, activation_e: int, device="cpu") -> torch.Tensor:
     """2^-(e + activation_e) per column (float32 [batch, N]): what a product of
     the scaled operands is multiplied by."""
-    e = row_exponents(_rows(data, offset, strides, batch, k, n, device))
-    return _power_of_two(-(e + activation_e))
+    return scales_of(column_exponents(data, offset, strides, batch, k, n, device), activation_e)
+
+
+def scales_of(exponents: torch.Tensor, activation_e: int) -> torch.Tensor:
+    return _power_of_two(-(exponents + activation_e))
+
+
+def scratch_bytes(elements: int, batch: int, k: int, n: int) -> int:
+    """Device memory that making a pair copy of a view of a constant of so many
+    elements takes beside the copy: the constant, at most six fp32 values per
+    element of a chunk, and per row a few words."""
+    kp = padded_k(k)
+    return 4 * elements + 24 * min(max(CHUNK, kp), batch * n * kp) + 64 * batch * n
 
 
 def pair_bytes(batch: int, k: int, n: int) -> int:

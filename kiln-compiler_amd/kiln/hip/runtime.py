@@ -117,11 +117,18 @@ def _on_pairs(name: str) -> bool:
     return "@f16:" in name or "@f16s:" in name
 
 
-def pair_constant(recipe, constants: dict, name: str, where) -> torch.Tensor:
-    """The fp16-pair copy of a weight, or its columns' scales, made on `where`."""
-    src, offset, strides, batch, k, n = recipe[:6]
+def pair_constant(recipe, constants: dict, name: str, where, made: dict) -> torch.Tensor:
+    """The fp16-pair copy of a weight, or its columns' scales, made on `where`.
+    made: exponents of the weights made before, so that a weight is read once
+    for both."""
+    src, offset, strides, batch, k, n = view = recipe[:6]
     args = (constants[src], offset, strides, batch, k, n)
-    return f16.pair_rows(*args, where) if "@f16:" in name else f16.column_scales(*args, recipe[6][1], where)
+    if "@f16:" in name:
+        copy, made[view] = f16.pair_copy(*args, where)
+        return copy
+    if view not in made:
+        made[view] = f16.column_exponents(*args, where)
+    return f16.scales_of(made[view], recipe[6][1])
 
 
 def host_constant(program, constants: dict, name: str) -> np.ndarray:
@@ -132,7 +139,7 @@ def host_constant(program, constants: dict, name: str) -> np.ndarray:
         return np.ascontiguousarray(constants[name], np.float32)
     src, offset, strides, batch, k, n = recipe[:6]
     if _on_pairs(name):
-        return pair_constant(recipe, constants, name, "cpu").numpy()
+        return pair_constant(recipe, constants, name, "cpu", {}).numpy()
     if "@nk:" in name:
         return nk_copy(constants[src], offset, strides, batch, k, n)
     if "@nkg:" in name or "@lnc:" in name or "@lng:" in name:
@@ -173,22 +180,28 @@ class HIPExecutable:
         # (fp16-pair copies are made on the device, below)
         host = [None if _on_pairs(name) else host_constant(program, constants, name) for name in program.consts]
         self.weight_bytes = sum(int(h.nbytes) for h in host if h is not None)
+        scratch = 0   # while a pair copy is made
         for name in program.consts:
             if _on_pairs(name):
-                batch, k, n = program.derived[name][3:6]
+                src, _, _, batch, k, n = program.derived[name][:6]
                 self.weight_bytes += f16.pair_bytes(batch, k, n) if "@f16:" in name else 4 * batch * n
+                scratch = max(scratch, f16.scratch_bytes(int(np.size(constants[src])), batch, k, n))
         self.arena_bytes = arena_bytes
         ws = self.plan.workspace_bytes
         outs = 4 * sum(int(np.prod(s)) for s in self.output_shapes)
-        check_memory(self.device, arena_bytes + self.weight_bytes + ws + outs,
-                     f"the arena ({arena_bytes / MiB:.1f} MiB), weights ({self.weight_bytes / MiB:.1f} MiB), "
+        check_memory(self.device, arena_bytes + self.weight_bytes + ws + outs + scratch,
+                     f"the arena ({arena_bytes / MiB:.1f} MiB), weights ({self.weight_bytes / MiB:.1f} MiB, "
+                     f"{scratch / MiB:.1f} MiB more while they are prepared), "
                      f"split-K workspace ({ws / MiB:.1f} MiB) and outputs")
         self.arena = torch.empty(max(arena_bytes, 256), dtype=torch.uint8, device=self.device)
         # every split-K launch writes all the partials it reads: no clearing
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=self.device) if ws else None
+        exponents = {}
         self.constants = [torch.from_numpy(h).to(self.device) if h is not None
-                          else pair_constant(program.derived[name], constants, name, self.device)
+                          else pair_constant(program.derived[name], constants, name, self.device, exponents)
                           for name, h in zip(program.consts, host)]
+        # pair copies are made by this stream's kernels; calls come on any stream
+        torch.cuda.current_stream(self.device).synchronize()
         self.plan.bind([c.data_ptr() for c in self.constants], self.arena.data_ptr(),
                        self.workspace.data_ptr() if ws else None, ws)
         self.guards = None

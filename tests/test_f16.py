@@ -395,3 +395,16 @@ def test_stored_plan_is_not_reused_with_another_mask(interpreting, tmp_path, mon
         with torch.no_grad():
             torch.testing.assert_close(c(x), model(x), rtol=3e-2, atol=3e-2, equal_nan=True)
     assert c.report.lowering["plan_cache"] == "stored"
+
+
+@pytest.mark.parametrize("batch,k,n", [(1, 40, 24), (3, 61, 5), (2, 8, 1)])
+@pytest.mark.parametrize("chunk", [1, 64, 200])
+def test_pair_copy_in_chunks_has_the_same_bits(batch, k, n, chunk):
+    # a transposed view at an offset, made whole and a few rows at a time;
+    # exponents and scales come from the same read of the weight
+    w = np.random.default_rng(1).standard_normal(7 + batch * k * n).astype(np.float32)
+    args = (w, 7, (k * n, 1, k), batch, k, n)
+    copy, exponents = f16.pair_copy(*args, chunk=chunk)
+    assert torch.equal(copy, f16.pair_rows(*args))
+    assert torch.equal(exponents, f16.column_exponents(*args))
+    assert torch.equal(f16.scales_of(exponents, 3), f16.column_scales(*args, 3))

@@ -198,3 +198,31 @@ def test_operand_that_is_also_the_residual(precision, tol):
     with torch.no_grad():
         ref = model.double()(x.double())
     np.testing.assert_allclose(out.double().numpy(), ref.numpy(), rtol=tol, atol=tol)
+
+
+def test_compile_returns_with_its_weights_made():
+    # weights are made by kernels of the stream that compiles; calls come on
+    # any stream, so nothing may be pending, and what is made beside the copy
+    # stays under the size that the memory check counts
+    from kiln.hip import f16
+
+    model = torch.nn.Sequential(torch.nn.LayerNorm(1024), torch.nn.Linear(1024, 8192, bias=False)).eval()
+    x = torch.randn(300, 1024)
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            c = kiln.compile(model, (x,), device="cuda", cuda_graphs=False)
+            assert stream.query()
+        xd = x.cuda()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            out = c(xd)
+        side.synchronize()
+        torch.testing.assert_close(out.cpu(), model(x).detach(), rtol=RTOL, atol=1e-4)
+    w = np.ones((1024, 8192), np.float32)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    copy, exponents = f16.pair_copy(w, 0, (0, 8192, 1), 1, 1024, 8192, "cuda")
+    peak = torch.cuda.max_memory_allocated() - before
+    assert peak <= f16.pair_bytes(1, 1024, 8192) + f16.scratch_bytes(w.size, 1, 1024, 8192)
