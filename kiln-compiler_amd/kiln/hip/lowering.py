@@ -467,6 +467,15 @@ class _Lowerer:
         if (buf.type.nbytes != 4 * math.prod(a.shape) or not self._reads_only(k, buf, [a])
                 or buf in self.g.results):
             return None
+        # the library's limits, which the fp32 configurations do not have:
+        # 32-bit byte offsets (A and B spans below 2^29 elements) and an
+        # operand for the column scales beside the epilogue's
+        m, kk, n = a.shape[-2], a.shape[-1], b.shape[-1]
+        if (m - 1) * lay.strides[-2] + kk >= 1 << 29 or n * f16.padded_k(kk) >= 1 << 29:
+            return None
+        read = {v for v in kernel_inputs(self.g, k) if v is not a and v is not b}
+        if 2 + len(read) + len(kernel_outputs(self.g, k, self.users)) + 1 > kl.MAX_REFS:
+            return None
         producer = self.g.kernel_of(buf.node)
         if producer is None or not self._writes_f16(producer, buf):
             return None

@@ -12,6 +12,7 @@ import torch.nn.functional as F
 import kiln
 import oracle
 from kiln.hip import autotune, f16
+from kiln.hip import lib as kl
 from kiln.hip.bounds import Bounds
 from kiln.hip.lowering import _Lowerer, lower_graph, operand_scales
 from models.transformer import Block, gpt2_init_
@@ -408,3 +409,39 @@ def test_pair_copy_in_chunks_has_the_same_bits(batch, k, n, chunk):
     assert torch.equal(copy, f16.pair_rows(*args))
     assert torch.equal(exponents, f16.column_exponents(*args))
     assert torch.equal(f16.scales_of(exponents, 3), f16.column_scales(*args, 3))
+
+
+# -- what the pair configurations refuse --------------------------------------------------------
+
+
+@pytest.mark.parametrize("m,on_pairs", [(699050, True), (699051, False)])
+def test_operands_of_2_29_elements_stay_off_pairs(m, on_pairs):
+    # rows of 768: (m - 1) * 768 + 768 below 2^29, the library's limit for
+    # 32-bit byte offsets, and above
+    from kiln.api import Options, build_passes
+    from kiln.passes.manager import PassManager
+
+    w, b = np.full((768, 64), 0.02, np.float32), np.zeros(64, np.float32)
+    g = autotune._linear_graph(1, m, 64, 768, w, b, True)
+    PassManager(build_passes(Options())).run(g)
+    prog = lower_graph(g)
+    assert ("f16x3" in prog.launches[-1].summary) == on_pairs
+    if not on_pairs:
+        kl.Plan([l.desc for l in prog.launches])   # the library takes it
+
+
+@pytest.mark.parametrize("residuals,on_pairs", [(7, True), (8, False)])
+def test_epilogue_that_fills_the_operand_table_stays_off_pairs(interpreting, residuals, on_pairs):
+    # a launch has 12 operands: the product's two, bias, residuals, output,
+    # and on pairs the column scales
+    torch.manual_seed(0)
+    ln, lin = torch.nn.LayerNorm(64).eval(), torch.nn.Linear(64, 48).eval()
+
+    def fn(x, *rs):
+        y = lin(ln(x))
+        for r in rs:
+            y = y + r
+        return y
+
+    c = check(fn, torch.randn(300, 64), *[torch.randn(300, 48) for _ in range(residuals)])
+    assert any("f16x3" in l.summary for l in c._exe.program.launches) == on_pairs
