@@ -83,19 +83,43 @@ inline uint16_t bf16_bits(float x) {
   return (uint16_t)((u + (((u >> 16) & 1u) + 0x7FFFu)) >> 16);
 }
 
+// A scaled value as its fp16 pair holds it (kh_common.hpp): h + l, infinite
+// halves where it overflows.
+inline float f16_pair(float x) {
+  const _Float16 h = (_Float16)x, l = (_Float16)(x - (float)h);
+  return (float)h + (float)l;
+}
+
 // Operand j at element `off`: fp32, or bf16 when the launch stores it as
 // bf16 (kh_launch.cfg[7]), read widened and written rounded to nearest even
-// as the kernels do.
+// as the kernels do. An output stored as fp16 pairs is written as the fp32
+// value of the pair, scaled: its readers (products and attention on pairs)
+// take back the scale, so a plan whose scales overflow, lose bits or do not
+// match shows it here. (bf16 pair words are written as plain fp32: the reader
+// splits them.)
 struct Operands {
   float *const *p;
-  uint32_t m16;
-  Operands(const kh_launch &L, float *const *ptrs) : p(ptrs), m16(bf16_refs(L)) {}
+  uint32_t m16, pairs;
+  float scale;
+  Operands(const kh_launch &L, float *const *ptrs)
+      : p(ptrs), m16(bf16_refs(L)), pairs(f16_pair_outputs(L)), scale(L.fparams[3]) {}
+  // Outputs that the launch stores as fp16 pairs: of a ROW or ATTN launch
+  // cfg[6] says so, of a product its precision (an fp32 plan's).
+  static uint32_t f16_pair_outputs(const kh_launch &L) {
+    const uint32_t mp = pair_refs(L);
+    switch (L.family) {
+      case KH_FAM_ROW: return L.cfg[6] == KH_PAIR_F16 ? mp : 0u;
+      case KH_FAM_ATTN: return L.cfg[6] == KH_PAIR_F16 ? mp & 8u : 0u;
+      case KH_FAM_GEMM: return L.cfg[3] == KH_PREC_F16X3 || L.cfg[3] == KH_PREC_FP32 ? mp & ~3u : 0u;
+      default: return 0u;
+    }
+  }
   float ld(int j, int64_t off) const {
     return (m16 >> j & 1) ? bf16_value(reinterpret_cast<const uint16_t *>(p[j])[off]) : p[j][off];
   }
   void st(int j, int64_t off, float v) const {
     if (m16 >> j & 1) reinterpret_cast<uint16_t *>(p[j])[off] = bf16_bits(v);
-    else p[j][off] = v;
+    else p[j][off] = (pairs >> j & 1) ? f16_pair(v * scale) : v;
   }
 };
 
@@ -210,15 +234,18 @@ void host_red(const kh_launch &L, float *const *p) {
 // scale mode and the mask mode. Fully masked rows give NaN, as eager does.
 // bf16 products (bf): q and k rounded to bf16 for the scores, the softmax
 // weights and v rounded to bf16 for the weighted sum (the two products of an
-// unfused attention whose matmuls take bf16 inputs).
+// unfused attention whose matmuls take bf16 inputs). On fp16 pairs q, k and v
+// are scaled, qk_inv and v_inv take that back; the kernel drops the products
+// of two low halves (2^-22) and splits the probabilities too, at 23 bits,
+// which is not modelled.
 void attend(int64_t tk, int64_t dh, int scale_mode, float scale, int mask_mode, int64_t query,
             const float *q, int64_t q_sd, const float *k, int64_t k_sj, int64_t k_sd, const float *v, int64_t v_sj,
-            int64_t v_sd, const float *mask, int64_t mask_sj, double *out, int prec = 0) {
+            int64_t v_sd, const float *mask, int64_t mask_sj, double *out, int prec = 0, float qk_inv = 1.0f,
+            float v_inv = 1.0f) {
   // one product of the two matmuls: fp32 inputs, bf16-rounded inputs, or the
   // three-pass sum lo.hi + hi.lo + hi.hi of the bf16 halves (a non-finite hi
   // keeps lo 0)
   auto prod = [prec](float x, float y) -> double {
-    // (fp16 pairs hold 23 bits of each input: taken as exact here)
     if (prec == 0 || prec == 3) return (double)x * (double)y;
     const float xh = bf16_round(x), yh = bf16_round(y);
     if (prec == 1) return (double)xh * (double)yh;
@@ -231,7 +258,7 @@ void attend(int64_t tk, int64_t dh, int scale_mode, float scale, int mask_mode, 
     float dot = 0.0f;
     double acc = 0.0;
     for (int64_t d = 0; d < dh; ++d) acc += prod(q[d * q_sd], k[j * k_sj + d * k_sd]);
-    dot = (float)acc;
+    dot = (float)(acc * qk_inv);
     if (scale_mode == KH_ATTN_SCALE_MUL) dot *= scale;
     if (scale_mode == KH_ATTN_SCALE_DIV) dot /= scale;
     if (mask_mode == KH_ATTN_MASK_CAUSAL && j > query) dot = -INFINITY;
@@ -247,7 +274,7 @@ void attend(int64_t tk, int64_t dh, int scale_mode, float scale, int mask_mode, 
     double acc = 0.0;
     for (int64_t j = 0; j < tk; ++j)
       acc += prec == 1 || prec == 2 ? prod((float)(s[j] / l), v[j * v_sj + d * v_sd]) : s[j] * (double)v[j * v_sj + d * v_sd];
-    out[d] = prec == 1 || prec == 2 ? acc : acc / l;
+    out[d] = prec == 1 || prec == 2 ? acc : acc / l * v_inv;
   }
 }
 
@@ -276,7 +303,8 @@ void host_attn(const kh_launch &L, float *const *p0) {
                                                        : nullptr;
       attend(tk, dh, L.cfg[1], L.fparams[0], L.cfg[0], i, p[0] + b * Q.strides[0] + i * Q.strides[1], Q.strides[2],
              p[1] + b * K.strides[0], K.strides[1], K.strides[2], p[2] + b * V.strides[0], V.strides[1], V.strides[2],
-             mask, mask ? L.refs[4].strides[2] : 0, out.data(), L.cfg[5]);
+             mask, mask ? L.refs[4].strides[2] : 0, out.data(), L.cfg[5], L.cfg[5] == 3 ? L.fparams[1] : 1.0f,
+             L.cfg[5] == 3 ? L.fparams[2] : 1.0f);
       for (int64_t d = 0; d < dh; ++d)
         Operands(L, p).st(3, b * O.strides[0] + i * O.strides[1] + d * O.strides[2], (float)out[d]);
     }
@@ -336,9 +364,6 @@ void host_matmul(const kh_launch &L, float *const *p) {
   for (int64_t b = 0; b < batch; ++b)
     for (int64_t m = 0; m < M; ++m) {
       a_row(L, p, b, m, row);
-      // fp16 pairs: an activation's pair storage is its fp32 value here, split as its producer would
-      if (prec == KH_PREC_F16X3)
-        for (float &x : row) x *= L.fparams[0];
       for (int64_t n = 0; n < N; ++n) {
         double acc = 0.0;
         for (int64_t k = 0; k < K; ++k) {
@@ -348,7 +373,8 @@ void host_matmul(const kh_launch &L, float *const *p) {
             acc += (double)a * (double)p[1][at];
           } else if (prec == KH_PREC_BF16) {
             acc += (double)bf16_round(a) * (double)bf16_value(b16[at]);
-          } else if (prec == KH_PREC_F16X3) {   // fp16 pairs: l.h + h.l + h.h, B in blocks of 8 h and 8 l
+          } else if (prec == KH_PREC_F16X3) {
+            // fp16 pairs: l.h + h.l + h.h, A scaled by its producer (Operands), B in blocks of 8 h and 8 l
             const _Float16 *w = reinterpret_cast<const _Float16 *>(p[1]) + 2 * (at - k % 8) + k % 8;
             const double wh = (double)w[0], wl = (double)w[8];
             const _Float16 ah = (_Float16)a, al = (_Float16)(a - (float)ah);

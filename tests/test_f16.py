@@ -445,3 +445,50 @@ def test_epilogue_that_fills_the_operand_table_stays_off_pairs(interpreting, res
 
     c = check(fn, torch.randn(300, 64), *[torch.randn(300, 48) for _ in range(residuals)])
     assert any("f16x3" in l.summary for l in c._exe.program.launches) == on_pairs
+
+
+# -- what the host interpreter sees of pairs ------------------------------------------------------
+
+
+@pytest.mark.parametrize("q,v", [(1.0, 1.0), (32.0, 32.0), (2.0 ** -9, 2.0 ** -12), (2.0 ** 9, 2.0 ** 12)])
+def test_interpreted_attention_on_pairs(interpreting, q, v):
+    # q and k of very different size (the scores stay), v large and small: each
+    # in its own buffer with its own scale
+    torch.manual_seed(0)
+    model = _Projected(64, 2).eval()
+    with torch.no_grad():
+        for lin, s in ((model.q, q), (model.k, 1.0 / q), (model.v, v)):
+            lin.weight.mul_(s), lin.bias.mul_(s)
+    c = kiln.compile(model, (torch.randn(192, 64),), device="cuda")
+    assert any("products:f16x3" in l.summary for l in c._exe.program.launches)
+    err, eager, _ = _errors(model, torch.randn(192, 64))
+    assert err <= eager
+
+
+@pytest.mark.parametrize("factor,loses", [(4096.0, "range"), (2.0 ** -30, "bits")])
+def test_interpreter_sees_stale_scales(interpreting, tmp_path, monkeypatch, factor, loses):
+    # a plan with another model's scales of q, k and v: values past fp16's
+    # range are not finite, values far below it lose their bits
+    from kiln.hip import lowering
+
+    monkeypatch.setenv("KILN_CACHE_DIR", str(tmp_path))
+    monkeypatch.setattr(lowering, "constant_facts", lambda *_: "")
+    torch.manual_seed(0)
+    model, x = SelfAttention(64, 2).eval(), torch.randn(192, 64)
+    kiln.compile(model, (x,), device="cuda")
+    with torch.no_grad():
+        model.qkv.weight[128:] *= factor
+        model.qkv.bias[128:] *= factor
+    c = kiln.compile(model, (x,), device="cuda")
+    assert c.report.lowering["plan_cache"] == "stored"
+    out = c(x)
+    with torch.no_grad():
+        ref = copy.deepcopy(model).double()(x.double())
+    if loses == "range":
+        assert not torch.isfinite(out).all()
+    else:
+        assert float((out.double() - ref).norm() / ref.norm()) > 1e-3
+    monkeypatch.undo()
+    monkeypatch.setenv("KILN_HIP_INTERPRET", "1")
+    fresh = kiln.compile(model, (x,), device="cuda", plan_cache=False)(x)
+    assert float((fresh.double() - ref).norm() / ref.norm()) < 1e-6
