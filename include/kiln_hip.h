@@ -212,15 +212,17 @@ typedef struct kh_pass {
  * direct epilogue without split-K.
  * fp16 pairs: an fp32 product on KH_PREC_F16X3 configurations (101-110) reads
  * A and B as fp16 pairs: each value, scaled by a power of two into fp16's
- * range, as h = fp16(x) and l = fp16(x - h), a row in blocks of 8 values (16
- * bytes of h, then 16 bytes of l), 4 bytes a value, strides and offsets
- * counted in values and multiples of 8. A . B is taken as l.h + h.l + h.h in
- * fp32. A must be pair-stored (bit 16 of cfg[7]) with scale fparams[0]; B is
- * the [batch][N][K'] copy (K' a multiple of 8, zero padded); refs[cfg[5]],
- * strides 0 over M and 1 over N, is 1 / (scale of A * scale of column n),
- * applied before the epilogue. A direct epilogue's output may be pair-stored
- * too (also of an fp32 small-M configuration), a LayerNorm's and a blocked
- * attention's with cfg[6] = KH_PAIR_F16: scaled by fparams[3]. Scales are
+ * range, as h = fp16(x) and l = fp16(x - h), in B; a pair-stored activation (A
+ * here, q, k, v, outputs) holds l = fp16((x - h) 2^11), which keeps its bits
+ * where h is small. A row is in blocks of 8 values (16 bytes of h, then 16
+ * bytes of l), 4 bytes a value, strides and offsets counted in values and
+ * multiples of 8. A . B is taken as l.h + h.l + h.h in fp32. A must be
+ * pair-stored (bit 16 of cfg[7]) with scale fparams[0]; B is the
+ * [batch][N][K'] copy (K' a multiple of 8, zero padded); refs[cfg[5]], strides
+ * 0 over M and 1 over N, is 1 / (scale of A * scale of column n), applied
+ * before the epilogue. A direct epilogue's output may be pair-stored too (also
+ * of an fp32 small-M configuration), a LayerNorm's and a blocked attention's
+ * with cfg[6] = KH_PAIR_F16: scaled by fparams[3]. Scales are
  * powers of two; the caller guarantees that scaled values stay below 65504.
  */
 typedef struct kh_launch {

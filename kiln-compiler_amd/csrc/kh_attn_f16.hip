@@ -17,13 +17,15 @@
 //   * the probabilities' pairs are scaled by 2^14, so that p >= 2^-15 of the
 //     row's largest splits into a full pair.
 // Two workgroups of four waves per CU (64 KB of LDS each), two waves per SIMD.
-// Measured (12 heads of 64, causal; fp32 products before): T = 512 12.0 -> 8.4
-// us, 777 23.4 -> 12.1, 1024 27.0 -> 14.7, 2048 73.7 -> 36.2; 8 heads x 600
-// queries and keys, no mask, 21.9 -> 9.7. Error against float64 the same or
-// smaller. At T = 2048, with the copies left out 27.6 us and with softmax and
-// LDS reads left out too 21.9: the matrix cores' own time at the clock they
-// hold, the tail of the causal grid and the launch; each block is copied by
-// every query block that reads it (16 KB for 24 MFMAs).
+// Measured (12 heads of 64, causal; fp32 products before): T = 512 12.0 -> 7.9
+// us, 777 23.4 -> 11.1, 1024 27.0 -> 13.2, 2048 73.7 -> 34.0; 8 heads x 600
+// queries and keys, no mask, 21.9 -> 9.2. Error against float64 the same or
+// smaller. l halves stored times 2^11 cost 8 packed products a key block (the
+// probabilities' h times 2^-11) and the softmax's splits give them back: each
+// half one fused operation, 318 instructions a block against 332 with plain
+// halves. At T = 2048 the matrix cores' own time is about 22 us at the clock
+// they hold (copies, LDS reads and softmax left out, plain halves); each block
+// is copied by every query block that reads it (16 KB for 24 MFMAs).
 #include <type_traits>
 
 #include "kh_attn_args.hpp"
@@ -83,20 +85,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   const uint32_t flip = c < 0.0f ? 0x80008000u : 0u;
   c = fabsf(c);
 
-  // Q operands: block 2 i + half of the lane's query row
-  f16x8_t qf[NC][2];
-  {
-    const float *qp = a.q + b * a.q_b + (int64_t)min(qi, a.tq - 1) * a.q_t + 8 * half;
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        uint4 x = *reinterpret_cast<const uint4 *>(qp + 16 * i + 4 * p);
-        x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
-        qf[i][p] = __builtin_bit_cast(f16x8_t, x);
-      }
-  }
-
   const bool causal = a.mask_mode == KH_ATTN_MASK_CAUSAL;
   const int kend = causal ? min(a.tk, q0 + kQB) : a.tk;
   const int nkb = (kend + kKB - 1) / kKB;
@@ -152,7 +140,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     asm volatile("" ::: "memory");
   };
   constexpr std::integral_constant<int, 0> kAll{};
-  constexpr std::integral_constant<int, NI> kAllButOneBlock{};
 
   // K operand (chunk i, half p): chunk 4 i + 2 half + p of row col
   const uint32_t k_at = k_lds + (uint32_t)col * RB + (uint32_t)((2 * half) ^ swz_kv<DH>(col)) * 16u;
@@ -187,6 +174,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
   };
 
+  // Q operands: block 2 i + half of the lane's query row: h, l, and h 2^-11 for
+  // K's l halves, which are stored times 2^11 as all activations' are. (Scores
+  // need q and k in absolute terms only: l and h 2^-11 may be subnormal.) Read
+  // behind the first block's copies, so that one memory latency covers both.
+  f16x8_t qf[NC][3];
+  auto form_q = [&] {
+    const float *qp = a.q + b * a.q_b + (int64_t)min(qi, a.tq - 1) * a.q_t + 8 * half;
+    uint4 raw[NC][2];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) raw[i][p] = *reinterpret_cast<const uint4 *>(qp + 16 * i + 4 * p);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        uint4 x = raw[i][p];
+        x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
+        qf[i][p] = __builtin_bit_cast(f16x8_t, x);
+      }
+      qf[i][1] = qf[i][1] * kPairDown;
+      qf[i][2] = qf[i][0] * kPairDown;
+    }
+  };
+
   // S^T block: register r of lane (col, half) = score of query col with key
   // (r / 4) * 8 + half * 4 + r % 4, the small products first; `between(i)`
   // is issued behind MFMA i
@@ -198,7 +210,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     for (int p = 0; p < 3; ++p)
 #pragma unroll
       for (int i = 0; i < NC; ++i) {
-        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i][p == 0], qf[i][p == 1], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i][p == 0], qf[i][2 - p], s, 0, 0, 0);
         between(p * NC + i);
       }
     return s;
@@ -238,11 +250,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const float m_new = fmaxf(m_run, kU ? mx : mx * c);
     const float m_use = m_new == -INFINITY ? 0.0f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float part[4];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       s[r] = __builtin_amdgcn_exp2f(kU ? s[r] - m_use : fmaf(s[r], c, -m_use));
-      part[r & 3] += s[r];
+      part[r & 3] = r < 4 ? s[r] : part[r & 3] + s[r];
     }
     const float2 sh = halves((part[0] + part[1]) + (part[2] + part[3]));
     l_run = fmaf(l_run, alpha, sh.x + sh.y);
@@ -255,17 +267,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       uint4 h, l;
-      split_f16x2(p[8 * i] * kUp, p[8 * i + 1] * kUp, h.x, l.x);
-      split_f16x2(p[8 * i + 2] * kUp, p[8 * i + 3] * kUp, h.y, l.y);
-      split_f16x2(p[8 * i + 4] * kUp, p[8 * i + 5] * kUp, h.z, l.z);
-      split_f16x2(p[8 * i + 6] * kUp, p[8 * i + 7] * kUp, h.w, l.w);
+      split_f16x2(p[8 * i], p[8 * i + 1], kUp, h.x, l.x);
+      split_f16x2(p[8 * i + 2], p[8 * i + 3], kUp, h.y, l.y);
+      split_f16x2(p[8 * i + 4], p[8 * i + 5], kUp, h.z, l.z);
+      split_f16x2(p[8 * i + 6], p[8 * i + 7], kUp, h.w, l.w);
       const f16x8_t ph = __builtin_bit_cast(f16x8_t, h), pl = __builtin_bit_cast(f16x8_t, l);
+      const f16x8_t pd = ph * kPairDown;   // (V's l halves are stored times 2^11)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][1], ph, oacc[t], 0, 0, 0);
+      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][0], ph, oacc[t], 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][0], pl, oacc[t], 0, 0, 0);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][0], ph, oacc[t], 0, 0, 0);
+      for (int t = 0; t < NT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i][t][1], pd, oacc[t], 0, 0, 0);
     }
   };
 
@@ -278,7 +291,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     f16x8_t kf[NC][2], vf[2][NT][2];
     copy_k(kb);
     copy_v(kb);
-    landed(kAllButOneBlock);
+    form_q();
+    landed(kAll);
     read_k(kf);
     lds_reads_done();
     copy_k(min(kb + NW, nkb - 1));

@@ -279,30 +279,42 @@ __device__ __forceinline__ void split_bf16x8(const float4 &x, const float4 &y, b
 // them). A product of two pairs is h.h + h.l + l.h in three fp16 MFMAs with
 // fp32 accumulation; the dropped l.l is below 2^-22 of the product.
 //
+// Weights are held so, each column with a power of two of its own.
+// Activations share one power of two, chosen for their upper bound, and a row
+// may lie far below that (a LayerNorm's row whose spread is small against
+// sqrt(eps)), so their l is stored times 2^11: it becomes subnormal no earlier
+// than h does, and |x - h - l 2^-11| <= 2^-23 |x| holds down to |x| = 2^-13,
+// <= 2^-36 below. Readers multiply l by the other operand's h 2^-11 (kPairDown).
+//
 // Storage of a row of pairs (32-byte aligned, 4 bytes a value as in fp32):
 // blocks of 8 values, 16 bytes of h then 16 bytes of l, so an MFMA operand of
 // 8 consecutive values is one 128-bit read per half.
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+// Two values times `scale` (a power of two) as the words of their h halves and
+// of their l halves, these times UP (1, or 2^11 for pair storage of
+// activations). The difference to h and its product with UP are exact, so each
+// half is one fused operation that rounds to fp16; kept in one word, h is not
+// computed a second time for l.
+template <int UP = 1>
+__device__ __forceinline__ void split_f16x2(float x, float y, float scale, uint32_t &h, uint32_t &l) {
   typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-  f16x2_t r;
-  r[0] = (_Float16)a, r[1] = (_Float16)b;
-  return __builtin_bit_cast(uint32_t, r);
+  h = __builtin_bit_cast(uint32_t, f16x2_t{(_Float16)fmaf(x, scale, 0.0f), (_Float16)fmaf(y, scale, 0.0f)});
+  asm("" : "+v"(h));
+  const f16x2_t hh = __builtin_bit_cast(f16x2_t, h);
+  auto low = [&](float v, _Float16 hv) {
+    if constexpr (UP == 1) return (_Float16)fmaf(v, scale, -(float)hv);
+    else return (_Float16)fmaf((float)hv, -(float)UP, v * (scale * (float)UP));
+  };
+  l = __builtin_bit_cast(uint32_t, f16x2_t{low(x, hh[0]), low(y, hh[1])});
 }
-
-// Two (scaled) values as the words of their h halves and of their l halves.
-__device__ __forceinline__ void split_f16x2(float x, float y, uint32_t &h, uint32_t &l) {
-  const _Float16 hx = (_Float16)x, hy = (_Float16)y;
-  h = pack_f16x2(x, y);
-  l = pack_f16x2(x - (float)hx, y - (float)hy);
-}
+constexpr _Float16 kPairDown = (_Float16)0x1p-11f;
 
 // Columns [n, n + 4) (n a multiple of 4) of a row of pairs: v * scale.
 __device__ __forceinline__ void store_f16_pairs4(float *row, int64_t n, const float4 &v, float scale) {
   uint2 h, l;
-  split_f16x2(v.x * scale, v.y * scale, h.x, l.x);
-  split_f16x2(v.z * scale, v.w * scale, h.y, l.y);
+  split_f16x2<2048>(v.x, v.y, scale, h.x, l.x);
+  split_f16x2<2048>(v.z, v.w, scale, h.y, l.y);
   char *block = reinterpret_cast<char *>(row) + (n >> 3) * 32 + (n & 4) * 2;
   *reinterpret_cast<uint2 *>(block) = h;
   *reinterpret_cast<uint2 *>(block + 16) = l;

@@ -7,9 +7,12 @@
 //
 // Same contract as the rest of the matmul family (the reference's tl.dot
 // kernel with fused epilogue, kiln/gpu/codegen.py:484-530). The fp32 MFMA
-// runs at 157 TFLOP/s; three fp16 passes are worth 840, and hold every
-// operand to 23 bits (error against float64 below that of the fp32 MFMA
-// products, whose sums round once per four terms instead of once per 32).
+// runs at 157 TFLOP/s; three fp16 passes are worth 840. Operands keep 23 bits
+// where the plan sends a product here: activations down to 2^-27 of the bound
+// their scale is chosen for, weights down to 2^-15 of their column's largest
+// (kh_common.hpp, kiln/hip/bounds.py). On GPT-2 blocks the error against
+// float64 is below that of the fp32 MFMA products, whose sums round once per
+// four terms instead of once per 32.
 //
 // A pair row has the bytes of an fp32 row, and an MFMA operand (8 consecutive
 // K values of one row) is one 16-byte chunk of h and one of l, so the LDS
@@ -73,12 +76,14 @@ void gemm_f16_kernel(const GemmArgs a) {
   constexpr int A_WORDS = BM * BK, STAGE = (BM + BN) * BK;
   constexpr int A_PER_WAVE = BM * CH / 64 / kWaves, B_PER_WAVE = BN * CH / 64 / kWaves;
   constexpr int COPIES = A_PER_WAVE + B_PER_WAVE;
-  // DUAL: the small products (l.h, h.l) accumulate apart from h.h and join it
-  // at the end, so two thirds of the roundings happen at 2^-11 of the sum's
-  // size (K = 768: error 3.2e-7 -> 1.9e-7 of the result, the fp32 MFMA chain
-  // 5.0e-7). Not where two waves per SIMD leave no registers for it.
-  constexpr bool DUAL = kWaves == 4 || FM * FN <= 8;
-  constexpr int ACCS = DUAL ? 2 : 1;
+  // SPLIT: the small products (b.l a.h, b.h a.l) accumulate apart from h.h and
+  // join it at the end, so two thirds of the roundings happen at 2^-11 of the
+  // sum's size (K = 768: error 3.2e-7 -> 1.9e-7 of the result, the fp32 MFMA
+  // chain 5.0e-7), and apart from each other: A's l halves are stored times
+  // 2^11. Not where two waves per SIMD leave no registers for it (92 spilled
+  // with one more set): there B's h is multiplied by 2^-11 for that pass.
+  constexpr bool SPLIT = kWaves == 4 || FM * FN <= 8;
+  constexpr int ACCS = SPLIT ? 3 : 1;
   constexpr int CS = TN + 4;   // TAPE staging row stride (floats, 16-byte aligned rows)
   static_assert(TM % MT == 0 && TN % MT == 0, "wave tile of whole MFMA blocks");
   static_assert((BM * CH) % (64 * kWaves) == 0 && (BN * CH) % (64 * kWaves) == 0, "copy mapping");
@@ -165,24 +170,27 @@ void gemm_f16_kernel(const GemmArgs a) {
   auto &acc = accs[0];
   // the MFMAs of one column block in one pass: l.h, h.l, then h.h (the small
   // products first; a block's three passes are FM x FN MFMAs apart)
+  f16x8_t down;   // !SPLIT: B's h times 2^-11 for the next group
   auto mfma_group = [&](int q, const Frags &f) {
     const int p = q / FN, fn = q % FN;
+    const f16x8_t b = p == 1 && !SPLIT ? down : f.b[fn][p == 0];
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm) {
-      f32x4 &c = accs[DUAL && p < 2 ? ACCS - 1 : 0][fm][fn];
-      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[fn][p == 0], f.a[fm][p == 1], c, 0, 0, 0);
+      f32x4 &c = accs[SPLIT ? 2 - p : 0][fm][fn];
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, f.a[fm][p == 1], c, 0, 0, 0);
     }
+    if (!SPLIT && (q + 1) / FN == 1) down = f.b[(q + 1) % FN][0] * kPairDown;
   };
   auto mfmas = [&](const Frags &f) {
 #pragma unroll
     for (int q = 0; q < 3 * FN; ++q) mfma_group(q, f);
   };
   auto join = [&] {
-    if constexpr (DUAL) {
+    if constexpr (SPLIT) {
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn) acc[fm][fn] += accs[1][fm][fn];
+        for (int fn = 0; fn < FN; ++fn) acc[fm][fn] += accs[1][fm][fn] * (float)kPairDown + accs[2][fm][fn];
     }
   };
 

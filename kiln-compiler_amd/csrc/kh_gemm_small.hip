@@ -171,11 +171,11 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
     }
   }
 
-  f32x4 acc[FM][FN], acc_small[FM][FN];   // (acc_small: PREC 3)
+  f32x4 acc[FM][FN], acc_bl[FM][FN], acc_al[FM][FN];   // (acc_bl, acc_al: PREC 3)
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
-    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = acc_small[fm][fn] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = acc_bl[fm][fn] = acc_al[fm][fn] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto part = [](const float4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
 
   for (int p = 0; p < NS - 1 && p < n_steps; ++p) issue(p);
@@ -271,14 +271,15 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
         }
     } else if constexpr (PREC == 3) {
       // chunk 2g is h, chunk 2g + 1 is l; the small products accumulate apart
-      // (their roundings are then 2^-11 of the sum's)
+      // (their roundings are then 2^-11 of the sum's) and apart from each
+      // other (A's l halves are stored times 2^11)
 #pragma unroll
       for (int p = 0; p < 3; ++p)
 #pragma unroll
         for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn) {
-            f32x4 &c = p < 2 ? acc_small[fm][fn] : acc[fm][fn];
+            f32x4 &c = p == 0 ? acc_al[fm][fn] : p == 1 ? acc_bl[fm][fn] : acc[fm][fn];
             c = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8_t *>(&xa[fm][p == 0]),
                                                        *reinterpret_cast<const f16x8_t *>(&xb[fn][p == 1]), c, 0, 0, 0);
           }
@@ -337,7 +338,9 @@ __global__ __launch_bounds__(64 * WK) void gemm_small_kernel(const GemmArgs a) {
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mine[(fm * MT + 4 * g + i) * CS + fn * MT + li] = acc[fm][fn][i] + (PREC == 3 ? acc_small[fm][fn][i] : 0.0f);
+      for (int i = 0; i < 4; ++i)
+        mine[(fm * MT + 4 * g + i) * CS + fn * MT + li] =
+            acc[fm][fn][i] + (PREC == 3 ? fmaf(acc_al[fm][fn][i], (float)kPairDown, acc_bl[fm][fn][i]) : 0.0f);
   if constexpr (LN) {
     // the row's statistics over this wave's K range: lanes li, li + 16,
     // li + 32, li + 48 merged (lane group 0's result kept)

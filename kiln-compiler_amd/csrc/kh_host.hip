@@ -83,11 +83,11 @@ inline uint16_t bf16_bits(float x) {
   return (uint16_t)((u + (((u >> 16) & 1u) + 0x7FFFu)) >> 16);
 }
 
-// A scaled value as its fp16 pair holds it (kh_common.hpp): h + l, infinite
-// halves where it overflows.
+// A scaled value as an activation's fp16 pair holds it (kh_common.hpp): h and
+// l 2^11, infinite halves where it overflows.
 inline float f16_pair(float x) {
-  const _Float16 h = (_Float16)x, l = (_Float16)(x - (float)h);
-  return (float)h + (float)l;
+  const _Float16 h = (_Float16)x, l = (_Float16)((x - (float)h) * 0x1p11f);
+  return (float)h + (float)l * 0x1p-11f;
 }
 
 // Operand j at element `off`: fp32, or bf16 when the launch stores it as
@@ -374,11 +374,12 @@ void host_matmul(const kh_launch &L, float *const *p) {
           } else if (prec == KH_PREC_BF16) {
             acc += (double)bf16_round(a) * (double)bf16_value(b16[at]);
           } else if (prec == KH_PREC_F16X3) {
-            // fp16 pairs: l.h + h.l + h.h, A scaled by its producer (Operands), B in blocks of 8 h and 8 l
+            // fp16 pairs: l.h + h.l + h.h, A scaled by its producer (Operands), B in blocks of 8 h and 8 l;
+            // A's l meets h 2^-11 rounded to fp16, as the 128x192 tile forms it
             const _Float16 *w = reinterpret_cast<const _Float16 *>(p[1]) + 2 * (at - k % 8) + k % 8;
             const double wh = (double)w[0], wl = (double)w[8];
-            const _Float16 ah = (_Float16)a, al = (_Float16)(a - (float)ah);
-            acc += (double)al * wh + (double)ah * wl + (double)ah * wh;
+            const _Float16 ah = (_Float16)a, al = (_Float16)((a - (float)ah) * 0x1p11f);
+            acc += (double)al * (double)(_Float16)((float)w[0] * 0x1p-11f) + (double)ah * wl + (double)ah * wh;
           } else {   // three products of bf16 halves: lo*hi + hi*lo + hi*hi
             const float a_hi = bf16_round(a);
             const float a_lo = std::isfinite(a_hi) ? bf16_round(a - a_hi) : 0.0f;

@@ -12,18 +12,17 @@ of it, both answered here from the graph and its constants:
     ReLU, tanh do not enlarge. A graph input has none.
 
   * Tight: the values lie close enough under that bound. A pair holds 23 bits
-    of a value near the bound but has an absolute floor, PAIR_FLOOR of the
-    bound, and a bound grows by sqrt(N) per product that no LayerNorm follows,
-    or with one outlier gain, where the values do not. So beside the bound goes
-    each element's usual size: |gamma|, |beta| behind a LayerNorm (whose rows
-    have norm sqrt(C)), root sums of squares through products and additions,
-    half behind GELU and ReLU, a mean of `keys` independent values behind
+    of a value near the bound but has an absolute floor (TIGHT below), and a
+    bound grows by sqrt(N) per product that no LayerNorm follows, or with one
+    outlier gain, where the values do not. So beside the bound goes each
+    element's usual size: |gamma|, |beta| behind a LayerNorm (whose rows have
+    norm sqrt(C)), root sums of squares through products and additions, half
+    behind GELU and ReLU, a mean of `keys` independent values behind
     attention. A product takes pairs only where, for every output column, the
-    floor stays a fraction of the rounding that fp32 operands of that size
-    bring anyway (2^-25 each); elsewhere it stays on the fp32 matrix cores. A
-    size is only claimed where it follows from the graph (an unknown one
-    refuses). Cancellation needs no care: what cancels has been rounded in fp32
-    before, relative to the terms.
+    bound is within TIGHT of the root mean square of what the column sums;
+    elsewhere it stays on the fp32 matrix cores. A size is only claimed where
+    it follows from the graph (an unknown one refuses). Cancellation needs no
+    care: what cancels has been rounded in fp32 before, relative to the terms.
 
 Bounds are for finite values: a NaN stays a NaN in fp16, and no infinity
 arises within a finite bound (a non-finite constant gives no bound).
@@ -40,16 +39,16 @@ from kiln.hip import f16
 
 NONE = (math.inf, math.inf)   # (largest magnitude, largest L2 norm of a row along the last dim)
 
-# Rounding of fp32 operands (2^-25 of a value, root mean square about half
-# that), and what a pair adds below its 23 bits: of an activation
-# PAIR_FLOOR of the bound, of a weight WEIGHT_FLOOR of its column's largest.
-FP32_ROUNDING = 2.0 ** -25
-PAIR_FLOOR = 2.0 ** -39
-WEIGHT_FLOOR = 2.0 ** -39
-# The floor's share of that rounding that is let through. GPT-2 blocks of
-# 2048 tokens reach 0.05 (their output projection, behind attention); at 0.5
-# the product's error grows by an eighth at most.
-SHARE = 0.5
+# How far a bound may lie above the usual size. Below its 23 bits a pair adds,
+# to a weight, at most 2^-39 of its column's largest, to q or k in a score
+# 2^-39 of their bounds, to any other activation 2^-50 of its bound
+# (csrc/kh_common.hpp); fp32 operands of the usual size bring 2^-25 of it each.
+# At 2^13 the first two stay under half of that, and the third under 2^-12: a
+# row may be 2^11 times smaller than usual (a LayerNorm's, where its spread is
+# small against sqrt(eps)) before it is held less well. GPT-2 blocks of 2048
+# tokens reach 2^10.4 (their output projection, behind attention) and 2^5
+# elsewhere, where rows may be 2^19 times smaller.
+TIGHT = 2.0 ** 13
 
 
 @dataclass
@@ -100,10 +99,9 @@ class Bounds:
         q, k, v = (x.amin(dim=-2) for x in (q, k, v))
         dh = m.q.shape[-1]
         q, k = (x.expand(*x.shape[:-1], dh) for x in (q, k))
-        limit = SHARE * FP32_ROUNDING / PAIR_FLOOR
-        noise = (q * k).norm(dim=-1)
-        ok = (tops[0] * k.norm(dim=-1) <= limit * noise).all() and (tops[1] * q.norm(dim=-1) <= limit * noise).all()
-        return exponents if bool(ok) and bool((tops[2] <= limit * v).all()) else None
+        usual = TIGHT * (q * k).norm(dim=-1)
+        ok = (tops[0] * k.norm(dim=-1) <= usual).all() and (tops[1] * q.norm(dim=-1) <= usual).all()
+        return exponents if bool(ok) and bool((tops[2] <= TIGHT * v).all()) else None
 
     # -- upper bounds ----------------------------------------------------------------
 
@@ -278,11 +276,10 @@ class Bounds:
         squares = (w / unit.float().unsqueeze(-2)).square_()
         weighted = torch.stack([torch.ones_like(s), (s / s_top).square()]).float() @ squares   # [.., 2, N]
         norm = top * weighted[..., 0, :].double().sqrt()
-        noise = top * s_top * weighted[..., 1, :].double().sqrt()
-        bound = self.largest(a)
-        tight = bool((bound * norm * PAIR_FLOOR <= SHARE * FP32_ROUNDING * noise).all()) and bool(
-            (top * float(s.norm()) * WEIGHT_FLOOR <= SHARE * FP32_ROUNDING * noise).all()) and f16.columns_fit(top)
-        size = noise.unsqueeze(-2) if noise.dim() > 1 else noise
+        usual = top * s_top * weighted[..., 1, :].double().sqrt()
+        tight = (bool((self.largest(a) * norm <= TIGHT * usual).all())
+                 and bool((top * float(s.norm()) <= TIGHT * usual).all()) and f16.columns_fit(top))
+        size = usual.unsqueeze(-2) if usual.dim() > 1 else usual
         return _Product(float(norm.max()), size.reshape([1] * (rank - size.dim()) + list(size.shape)), tight)
 
 

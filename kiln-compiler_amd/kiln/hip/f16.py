@@ -1,7 +1,8 @@
 """fp16-pair copies of GEMM weights (fp32 products on the fp16 matrix cores).
 
-A value x is held as h = fp16(x * 2^e) and l = fp16(x * 2^e - h): 23 of its 24
-significant bits (csrc/kh_common.hpp). The library reads B as [batch][N][K']
+A weight x is held as h = fp16(x * 2^e) and l = fp16(x * 2^e - h): 23 of its
+24 significant bits, and 2^-39 of its column's largest weight below
+(csrc/kh_common.hpp; kiln/hip/bounds.py says which products take them). The library reads B as [batch][N][K']
 rows (K' = K rounded up to 8, zero padded), in blocks of 8 values: 16 bytes of
 h, then 16 bytes of l. Each output column n has its own power of two, which
 puts the column's largest weight just below 2^15; the product's epilogue

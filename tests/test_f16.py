@@ -465,7 +465,7 @@ def test_interpreted_attention_on_pairs(interpreting, q, v):
     assert err <= eager
 
 
-@pytest.mark.parametrize("factor,loses", [(4096.0, "range"), (2.0 ** -30, "bits")])
+@pytest.mark.parametrize("factor,loses", [(4096.0, "range"), (2.0 ** -45, "bits")])
 def test_interpreter_sees_stale_scales(interpreting, tmp_path, monkeypatch, factor, loses):
     # a plan with another model's scales of q, k and v: values past fp16's
     # range are not finite, values far below it lose their bits
@@ -492,3 +492,23 @@ def test_interpreter_sees_stale_scales(interpreting, tmp_path, monkeypatch, fact
     monkeypatch.setenv("KILN_HIP_INTERPRET", "1")
     fresh = kiln.compile(model, (x,), device="cuda", plan_cache=False)(x)
     assert float((fresh.double() - ref).norm() / ref.norm()) < 1e-6
+
+
+# -- rows far smaller than usual ------------------------------------------------------------------
+
+
+@pytest.mark.parametrize("spread", [1.0, 1e-3, 1e-5, 1e-6, 1e-7, 1e-8, 1e-9])
+@pytest.mark.parametrize("what", ["linear", "mlp", "values"])
+def test_small_rows_keep_their_precision(interpreting, spread, what):
+    # a LayerNorm's rows shrink where their spread is small against sqrt(eps)
+    # = 3e-3, and without biases so does everything behind them; the scale is
+    # one for all rows. (1e-9: 2^-21 of the usual size.)
+    torch.manual_seed(0)
+    if what == "values":
+        model = SelfAttention(64, 2)
+        torch.nn.init.zeros_(model.qkv.bias)
+    else:
+        layers = [torch.nn.LayerNorm(64), torch.nn.Linear(64, 64, bias=False)]
+        model = torch.nn.Sequential(*layers, *([torch.nn.GELU(), torch.nn.Linear(64, 64, bias=False)] if what == "mlp" else []))
+    err, eager, pairs = _errors(model.eval(), torch.randn(300, 64) * spread)
+    assert err <= eager and pairs >= 1

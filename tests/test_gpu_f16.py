@@ -2,6 +2,8 @@
 against float64 of the fp32 inputs at the fp32 suite's tolerance, and with an
 error no larger than an fp32 MFMA configuration's that sums K in one chain."""
 
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -226,3 +228,43 @@ def test_compile_returns_with_its_weights_made():
     copy, exponents = f16.pair_copy(w, 0, (0, 8192, 1), 1, 1024, 8192, "cuda")
     peak = torch.cuda.max_memory_allocated() - before
     assert peak <= f16.pair_bytes(1, 1024, 8192) + f16.scratch_bytes(w.size, 1, 1024, 8192)
+
+
+@pytest.mark.parametrize("spread", [1e-6, 1e-8])
+@pytest.mark.parametrize("tile", [101, 102, 103, 106, 107])
+def test_small_rows_keep_their_precision(tile, spread):
+    # LayerNorm rows 2^-11.6 and 2^-18.3 of the usual size (spread / sqrt(eps))
+    torch.manual_seed(5)
+    rows = 1100 if tile not in autotune.SMALL_M else 70
+    model = torch.nn.Sequential(torch.nn.LayerNorm(256), torch.nn.Linear(256, 200, bias=False)).eval()
+    x = torch.randn(rows, 256) * spread
+    errs = []
+    for t in (tile, FP32_CHAIN):
+        c = kiln.compile(model, (x,), device="cuda", cuda_graphs=False,
+                         gpu_matmul_config=lambda *_: {"tile": t, "splitk": 1})
+        assert ("f16x3" in c._exe.program.launches[-1].summary) == (t == tile)
+        ref = copy.deepcopy(model).double()(x.double()).detach()
+        errs.append(float((c(x).cpu().double() - ref).norm() / ref.norm()))
+    assert errs[0] <= 1.1 * errs[1], errs
+
+
+@pytest.mark.parametrize("mask", [None, "causal", "add"])
+def test_attention_on_small_rows_keeps_its_precision(mask, monkeypatch):
+    from kiln.hip import lowering
+
+    torch.manual_seed(6)
+    model, x = _Attention(128, 2, 333, mask, 0.125).eval(), torch.randn(333, 128) * 1e-8
+    torch.nn.init.zeros_(model.qkv.bias)
+    ref = copy.deepcopy(model).double()(x.double()).detach()
+    good = ~torch.isnan(ref)
+
+    def err():
+        c = kiln.compile(model, (x,), device="cuda", cuda_graphs=False, plan_cache=False)
+        out = c(x.cuda()).cpu().double()
+        return any("products:f16x3" in l.summary for l in c._exe.program.launches), float(
+            (out - ref)[good].norm() / ref[good].norm())
+
+    pairs, on_pairs = err()
+    monkeypatch.setattr(lowering._Lowerer, "f16_attention", lambda self, k: None)
+    _, plain = err()
+    assert pairs and on_pairs <= 1.1 * plain, (on_pairs, plain)
