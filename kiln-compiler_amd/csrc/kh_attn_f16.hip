@@ -26,6 +26,7 @@
 // halves. At T = 2048 the matrix cores' own time is about 22 us at the clock
 // they hold (copies, LDS reads and softmax left out, plain halves); each block
 // is copied by every query block that reads it (16 KB for 24 MFMAs).
+#include <cmath>
 #include <type_traits>
 
 #include "kh_attn_args.hpp"
@@ -52,7 +53,9 @@ __device__ __forceinline__ int swz_kv(int r) {
   else return (r >> 1) & 7;
 }
 
-template <int DH, int NW, bool ADD>
+// ADD: an additive mask. WIDE: scores may exceed kPlainScores in the base-2
+// domain (see softmax).
+template <int DH, int NW, bool ADD, bool WIDE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void attn_f16_kernel(const AttnArgs a) {
   constexpr int NT = DH / 32;        // 32-wide tiles of the head dimension in O^T
   constexpr int NC = DH / 16;        // 16-wide chunks of the head dimension in S^T
@@ -227,9 +230,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   constexpr float kUp = 16384.0f;
 
   // Online softmax of one block, in place (see attn_kernel); only a wave's
-  // last block can hold keys past the causal diagonal or the last key.
+  // last block can hold keys past the causal diagonal or the last key. An
+  // exponent s c - m, one fused operation, is off by the rounding of m = c
+  // max(s), the same for every key of the row: it cancels against l, but
+  // scales the probabilities by up to 2^(ulp(m) / 2), which overflows their
+  // pairs from m = 2^25 on and all of fp32 from 2^31. Where scores can get
+  // there (WIDE), s c is rounded first, as m is.
   auto softmax = [&](f32x16 &s, int kb, auto masked) {
-    constexpr bool kU = ADD || decltype(masked)::value;   // s holds u, not the raw scores
+    constexpr bool kU = ADD || WIDE || decltype(masked)::value;   // s holds u, not the raw scores
     const int room = lim - kb * kKB - half * 4;
     float mx = -INFINITY;
 #pragma unroll
@@ -240,6 +248,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
         u = fmaf(u, c, a.mask[b * a.m_b + (int64_t)min(qi, a.tq - 1) * a.m_q + (int64_t)key * a.m_k] * kLog2e);
       } else if constexpr (kU) {
         u *= c;
+        asm("" : "+v"(u));   // (not fused into the exponent's subtraction)
       }
       if constexpr (decltype(masked)::value) u = (r >> 2) * 8 + (r & 3) < room ? u : -INFINITY;
       s[r] = u;
@@ -368,12 +377,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 }  // namespace
 
 hipError_t launch_attn_f16(const AttnArgs &a, int dh, int nw, dim3 grid, hipStream_t stream) {
+  // the largest score (base 2) that scaled q and k of up to 2^15 can give (a
+  // plan's stay below 2^14; 65504 still keeps p below 2): below 2^22 p stays
+  // under 1.2 and 16 instructions a key block (of 334) are left out. GPT-2's
+  // initial weights allow 2^16.
+  constexpr double kPlainScores = 4194304.0, kLargest = 32768.0;
+  const double c = 1.4426950408889634 * std::fabs((double)a.qk_inv) *
+                   (a.scale_mode == KH_ATTN_SCALE_MUL   ? std::fabs((double)a.scale)
+                    : a.scale_mode == KH_ATTN_SCALE_DIV ? 1.0 / std::fabs((double)a.scale)
+                                                        : 1.0);
+  const bool wide = !(c * dh * kLargest * kLargest < kPlainScores);
 #define KH_ATTN_F16_LAUNCH(D, W)                                                                     \
   if (dh == D && nw == W) {                                                                          \
     if (a.mask_mode == KH_ATTN_MASK_ADD)                                                             \
-      hipLaunchKernelGGL((attn_f16_kernel<D, W, true>), grid, dim3(64 * W), 0, stream, a);          \
+      hipLaunchKernelGGL((attn_f16_kernel<D, W, true, false>), grid, dim3(64 * W), 0, stream, a);   \
+    else if (wide)                                                                                   \
+      hipLaunchKernelGGL((attn_f16_kernel<D, W, false, true>), grid, dim3(64 * W), 0, stream, a);   \
     else                                                                                             \
-      hipLaunchKernelGGL((attn_f16_kernel<D, W, false>), grid, dim3(64 * W), 0, stream, a);         \
+      hipLaunchKernelGGL((attn_f16_kernel<D, W, false, false>), grid, dim3(64 * W), 0, stream, a);  \
     return hipGetLastError();                                                                        \
   }
   KH_ATTN_F16_LAUNCH(64, 8)

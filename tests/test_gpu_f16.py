@@ -268,3 +268,30 @@ def test_attention_on_small_rows_keeps_its_precision(mask, monkeypatch):
     monkeypatch.setattr(lowering._Lowerer, "f16_attention", lambda self, k: None)
     _, plain = err()
     assert pairs and on_pairs <= 1.1 * plain, (on_pairs, plain)
+
+
+@pytest.mark.parametrize("tokens,heads,mask", [(192, 2, None), (333, 2, "causal"), (200, 4, "causal"), (200, 2, "add")])
+@pytest.mark.parametrize("gain", [2.0 ** 9, 2.0 ** 12, 2.0 ** 17])
+def test_attention_with_huge_scores(tokens, heads, mask, gain, monkeypatch):
+    # scores around gain^2 (up to 2^34, where fp32 tells scores 2^11 apart
+    # from equal ones): the softmax is one-hot and finite, as it is in fp32
+    from kiln.hip import lowering
+
+    torch.manual_seed(7)
+    model, x = _Attention(128, heads, tokens, mask, 0.125).eval(), torch.randn(tokens, 128)
+    with torch.no_grad():
+        for p in (model.qkv.weight, model.qkv.bias):
+            p[:256] *= gain
+            p[256:] *= gain      # (v shares the scale: kept as large)
+    c = kiln.compile(model, (x,), device="cuda", cuda_graphs=False, plan_cache=False)
+    assert any("products:f16x3" in l.summary for l in c._exe.program.launches)
+    out = c(x.cuda()).cpu().double()
+    monkeypatch.setattr(lowering._Lowerer, "f16_attention", lambda self, k: None)
+    plain = kiln.compile(model, (x,), device="cuda", cuda_graphs=False, plan_cache=False)(x.cuda()).cpu().double()
+    ref = copy.deepcopy(model).double()(x.double()).detach()
+    good = ~torch.isnan(ref)
+    assert torch.equal(torch.isfinite(out), good)
+    # rows whose two best keys lie apart by more than fp32's rounding of such
+    # scores agree; the share of the others is small (2^-10 of a unit's odds)
+    row_ok = lambda t: ((t - ref).abs() <= 1e-3 * gain).all(dim=-1) | ~good.all(dim=-1)
+    assert float(row_ok(out).float().mean()) >= min(0.97, float(row_ok(plain).float().mean()) - 0.02)
