@@ -62,6 +62,12 @@ ATTN_X3_MIN_GROUPS = 192
 # 2048 73.7 -> 36.2); below, the 16-query fp32 kernel spreads over more
 # workgroups (T = 128 4.9 against 5.2 us)
 ATTN_F16_MIN_KEYS = 160
+# fp32 products of more than autotune.SMALL_M_MAX rows run on fp16 pairs from
+# this depth on: sums of fewer terms round less than the pairs' 23 bits do
+# (LayerNorm -> Linear, 1100 rows, K = 32 / 64 / 96 / 128 / 256: error of pairs
+# 1.20 / 1.10 / 1.04 / 1.00 / 0.50 times the fp32 tile's; at 300 and 600 rows
+# 0.92 or less for any K, against the fp32 kernel with a LayerNorm prologue)
+F16_MIN_DEPTH = 128
 
 _UNARY_OP = {"neg": "neg", "exp": "exp", "tanh": "tanh", "sigmoid": "sigmoid", "relu": "relu",
              "rsqrt": "rsqrt", "sqrt": "sqrt", "erf": "erf", "copy": "mov"}
@@ -1330,11 +1336,14 @@ class _Lowerer:
     def _prefers_f16(self, k) -> bool:
         """Does matmul kernel k (an fp32 product) run on fp16 pairs? Wherever it
         can, except where it would take a LayerNorm as its prologue: that
-        saves a launch, and stays on the fp32 small-M kernel."""
+        saves a launch, and stays on the fp32 small-M kernel; and except
+        shallow products of many rows (F16_MIN_DEPTH)."""
         operand = self.f16_operand(k)
         if operand is None:
             return False
         m, kk = next(n for n in k.nodes if n.op == "matmul").inputs[0].shape[-2:]
+        if m > autotune.SMALL_M_MAX and kk < F16_MIN_DEPTH:
+            return False
         producer = self.g.kernel_of(operand[0].node)
         if m > LN_PROLOGUE_MAX_ROWS or kk > 1024 or producer.kind != "reduction":
             return True

@@ -512,3 +512,11 @@ def test_small_rows_keep_their_precision(interpreting, spread, what):
         model = torch.nn.Sequential(*layers, *([torch.nn.GELU(), torch.nn.Linear(64, 64, bias=False)] if what == "mlp" else []))
     err, eager, pairs = _errors(model.eval(), torch.randn(300, 64) * spread)
     assert err <= eager and pairs >= 1
+
+
+@pytest.mark.parametrize("rows,k,on_pairs", [(1025, 96, False), (1025, 128, True), (1024, 96, True)])
+def test_shallow_products_of_many_rows_stay_off_pairs(rows, k, on_pairs):
+    # (lower error on the fp32 tiles there)
+    model = torch.nn.Sequential(torch.nn.LayerNorm(k), torch.nn.Linear(k, 64)).eval()
+    _, prog = lowered(model, torch.randn(rows, k))
+    assert ("f16x3" in prog.launches[-1].summary) == on_pairs
