@@ -472,8 +472,9 @@ def counter_report(probe_json, dirs):
                    divides by GRBM_GUI_ACTIVE instead, which under per-dispatch
                    collection also counts the profiler's own dispatch overhead);
       busy_us    = SQ_BUSY_CYCLES / SHADER_ARRAYS at the 2.4 GHz engine clock;
-      mfma_flops = SQ_INSTS_VALU_MFMA_MOPS_{F32,BF16} x 512 (its MfmaFlops*),
-                   against the launch's algorithmic flops;
+      mfma_flops = SQ_INSTS_VALU_MFMA_MOPS_{F32,BF16,F16} x 512 (its
+                   MfmaFlops*), against the launch's algorithmic flops (3 for
+                   a product in three fp16 passes);
       wait       = SQ_WAIT_ANY / SQ_WAVE_CYCLES (share of wave time waiting
                    on anything: memory counters or a barrier);
       wait_inst  = SQ_WAIT_INST_ANY / SQ_WAVE_CYCLES (waiting for an
@@ -503,7 +504,8 @@ def counter_report(probe_json, dirs):
     for l, v in zip(probe["groups"], per_group):
         busy = v.get("SQ_BUSY_CYCLES", 0.0) / SHADER_ARRAYS
         util = v["SQ_VALU_MFMA_BUSY_CYCLES"] / (busy * SIMDS) if "SQ_VALU_MFMA_BUSY_CYCLES" in v and busy else None
-        mops = sum(v.get(c, 0.0) for c in ("SQ_INSTS_VALU_MFMA_MOPS_F32", "SQ_INSTS_VALU_MFMA_MOPS_BF16"))
+        mops = sum(v.get(c, 0.0) for c in ("SQ_INSTS_VALU_MFMA_MOPS_F32", "SQ_INSTS_VALU_MFMA_MOPS_BF16",
+                                            "SQ_INSTS_VALU_MFMA_MOPS_F16"))
         fl = mops * 512 / l["flops"] if l["flops"] and mops else None
         lines.append(f"{l['group']:34s} {busy / ENGINE_GHZ / 1e3:7.1f} {fmt(util):>9s} {fmt(fl, False) if fl is None else f'{fl:14.3f}':>14s} "
                      f"{fmt(ratio(v, 'SQ_WAIT_ANY', 'SQ_WAVE_CYCLES')):>7s} "
