@@ -12,8 +12,8 @@
 //   * K operands are 128-bit LDS reads; V^T operands (8 keys of one head
 //     dimension per lane) come from ds_read_b64_tr_b16, which transposes 4
 //     keys x 16 dimensions per 16 lanes, so V needs no transposed copy;
-//   * LDS chunks (16 bytes) of row r sit at c ^ swz_kv(r), free of bank
-//     conflicts for both reads;
+//   * LDS chunks (16 bytes) of row r sit at c ^ swz_kv(r), which spreads both
+//     reads over the banks (4.7% of LDS cycles lost to conflicts);
 //   * the probabilities' pairs are scaled by 2^14, so that p >= 2^-15 of the
 //     row's largest splits into a full pair.
 // Two workgroups of four waves per CU (64 KB of LDS each), two waves per SIMD.

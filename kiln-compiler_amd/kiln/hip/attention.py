@@ -22,9 +22,10 @@ the reference's pipeline, and only on this backend.
 
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
-import numpy as np
+import torch
 
 from kiln.hip import lib as kl
 from kiln.ir import ops
@@ -265,8 +266,10 @@ def causal_or_none(graph: Graph, mask, batch, tq, tk):
     and -inf above it (the frozen ``triu(-inf, 1)`` buffer), else None."""
     if mask is None or not graph.is_const(mask) or mask.type.rank == 0:
         return None
-    data = np.asarray(graph.const_data(mask), dtype=np.float32)
-    full = np.broadcast_to(data.reshape(mask.shape), (batch, tq, tk) if mask.type.rank == 3 else (tq, tk))
-    want = np.triu(np.full((tq, tk), -np.inf, np.float32), 1)
-    ok = np.array_equal(full, np.broadcast_to(want, full.shape))
+    shape = (batch, tq, tk) if mask.type.rank == 3 else (tq, tk)
+    full = torch.as_tensor(graph.const_data(mask), dtype=torch.float32).reshape(mask.shape).expand(shape)
+    # (the first query's row before the whole mask)
+    if tq and tk and not bool((full[..., 0, 0] == 0.0).all() and torch.isneginf(full[..., 0, 1:]).all()):
+        return None
+    ok = bool((full == torch.full((tq, tk), -math.inf).triu_(1)).all())
     return kl.ATTN_MASK_CAUSAL if ok else None

@@ -260,23 +260,24 @@ class Bounds:
         if w is None or w.dim() < 2 or not w.numel():
             return none
         w = w.transpose(-2, -1) if perm else w   # [.., K, N]
-        # columns scaled by their largest weight, so that squares neither
-        # overflow nor vanish; root sums of squares of the columns, plain and
-        # weighted by A's sizes, from one pass over the squares
+        # root sums of squares of the columns, plain and weighted by A's sizes,
+        # from one pass over the squares; columns whose squares could overflow
+        # or vanish are scaled by their largest weight first
         top = torch.maximum(w.amax(dim=-2), -w.amin(dim=-2)).double()
         if not bool(torch.isfinite(top).all()):
             return none
-        unit = torch.where(top > 0, top, torch.ones_like(top))
+        unit = torch.where((top > 0) & ((top < 1e-12) | (top > 1e12)), top, torch.ones_like(top))
+        scaled = bool((unit != 1).any())
         # the smallest size along the other dims, for every K
         s = self.size(a)
         while s.dim() > 1:
             s = s.amin(dim=0)
         s = s.expand(w.shape[-2])
         s_top = float(s.max()) or 1.0
-        squares = (w / unit.float().unsqueeze(-2)).square_()
+        squares = (w / unit.float().unsqueeze(-2)).square_() if scaled else w.square()
         weighted = torch.stack([torch.ones_like(s), (s / s_top).square()]).float() @ squares   # [.., 2, N]
-        norm = top * weighted[..., 0, :].double().sqrt()
-        usual = top * s_top * weighted[..., 1, :].double().sqrt()
+        norm = unit * weighted[..., 0, :].double().sqrt()
+        usual = unit * s_top * weighted[..., 1, :].double().sqrt()
         tight = (bool((self.largest(a) * norm <= TIGHT * usual).all())
                  and bool((top * float(s.norm()) <= TIGHT * usual).all()) and f16.columns_fit(top))
         size = usual.unsqueeze(-2) if usual.dim() > 1 else usual
